@@ -9,12 +9,14 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/les_hip.h"
 #include "les_kernels.h"
 #include "les_mixed.h"
+#include "les_sor_res.h"
 
 using namespace les;
 
@@ -69,6 +71,15 @@ struct les_handle {
   bool rhs_stale = false;     // F.rhs's interior is behind ra
   bool graph_resident = false;  // the captured step is a resident solve (its replays leave
                                 // sp_p_current and rhs_stale set)
+  // The chip-resident solve (les_sor_res.hip): its cut of this grid (tk == 0: none) and its
+  // device buffers, allocated by the first solve that uses them.
+  ResPlan rplan;
+  ResBuf rbuf;
+  bool sor_form_set = false;  // les_set_sor_tile chose the iteration's form
+  bool capturing = false;     // the step is being captured into the handle's graph
+  bool graph_chip = false;    // the captured step runs the chip-resident solve
+  long res_wait = RES_WAIT_TICKS;
+  int ncu = 0;
   // workgroup shapes of the point-wise stencil kernels (les_autotune; 0 = 64 x 4)
   int shp_velnw = 0, shp_sm = 0, shp_visc = 0;
 };
@@ -88,6 +99,70 @@ int fail(les_handle* h, int code, const std::string& msg) {
     if (e_ != hipSuccess)                                                                   \
       return fail((h), LES_E_HIP, std::string(#call) + ": " + hipGetErrorString(e_));      \
   } while (0)
+
+// The chip-resident solve wants all its workgroups on the device together, one per CU at most.
+// Handles whose solves could not be there at the same time take turns: while more than one of
+// them has used that solve and their workgroups together exceed the CUs, whoever launches next
+// makes its stream wait for the last launch of another one.  (Kernels of other programs are
+// not seen here; the solve itself falls back to its queue form when they keep it from fitting.)
+struct ResTurn {
+  std::mutex m;
+  int handles = 0, wgs = 0;
+  les_handle* last = nullptr;
+  hipStream_t last_st = nullptr;
+  hipEvent_t ev = nullptr;
+  bool recorded = false;
+};
+constexpr int RES_DEVICES = 64;
+ResTurn g_turn[RES_DEVICES];
+
+// Allocates the chip-resident solve's buffers on first use; false: the grid does not fit or
+// there is no memory (the other forms of the solve serve it).
+bool res_ready(les_handle* h) {
+  if (h->rplan.tk == 0) return false;
+  if (h->rbuf.ctl) return true;
+  if (h->capturing) return false;
+  ResTurn& T = g_turn[h->cfg.device];
+  std::lock_guard<std::mutex> lock(T.m);
+  if (!T.ev && hipEventCreateWithFlags(&T.ev, hipEventDisableTiming) != hipSuccess) T.ev = nullptr;
+  if (!T.ev || res_alloc(h->d, h->sp.nr, h->rplan, h->st, h->rbuf) != hipSuccess) {
+    (void)hipGetLastError();
+    h->rplan.tk = 0;
+    return false;
+  }
+  // the handles before this one may have launched without recording
+  if (T.last && !T.recorded) T.recorded = hipEventRecord(T.ev, T.last_st) == hipSuccess;
+  ++T.handles;
+  T.wgs += h->rplan.nwg();
+  return true;
+}
+
+void res_release(les_handle* h) {
+  if (!h->rbuf.ctl) return;
+  ResTurn& T = g_turn[h->cfg.device];
+  std::lock_guard<std::mutex> lock(T.m);
+  --T.handles;
+  T.wgs -= h->rplan.nwg();
+  if (T.last == h) {  // its stream has been waited for
+    T.last = nullptr;
+    T.recorded = false;
+  }
+  res_free(h->rbuf);
+}
+
+// 'launch' enqueues work with a chip-resident solve of h on stream st, in its turn
+template <class Launch>
+auto res_in_turn(les_handle* h, hipStream_t st, Launch&& launch) {
+  ResTurn& T = g_turn[h->cfg.device];
+  std::lock_guard<std::mutex> lock(T.m);
+  const bool share = T.handles > 1 && T.wgs > h->ncu;
+  if (share && T.last && T.last != h && T.recorded) (void)hipStreamWaitEvent(st, T.ev, 0);
+  auto r = launch();
+  T.last = h;
+  T.last_st = st;
+  T.recorded = share && hipEventRecord(T.ev, st) == hipSuccess;
+  return r;
+}
 
 // Bounds table: lo/hi offsets relative to (0, ip, jp, kp) per dimension.
 struct BoundSpec {
@@ -522,6 +597,9 @@ extern "C" int les_create(const les_config* cfg, les_handle** out) {
       }
     }
   }
+  if (hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, cfg->device) != hipSuccess)
+    return bail(LES_E_HIP);
+  if (cfg->device < RES_DEVICES) h->rplan = res_plan(h->d, h->sp.nr, h->ncu);
   h->resident_ok = cfg->precision == LES_PREC_FP32 && cfg->sum_order == LES_SUM_EXACT;
   if (cfg->sum_order == LES_SUM_REFERENCE) {
     const int nrt = (cfg->ip + 1) / 2;
@@ -539,6 +617,7 @@ extern "C" int les_destroy(les_handle* h) {
   if (h->gexec) hipGraphExecDestroy(h->gexec);
   if (h->graph) hipGraphDestroy(h->graph);
   if (h->st) hipStreamSynchronize(h->st);
+  res_release(h);
   for (int f = 0; f < LES_NFIELDS; ++f)
     if (h->fld[f]) hipFree(h->fld[f]);
   if (h->mask) hipFree(h->mask);
@@ -899,6 +978,28 @@ bool use_split(const les_handle* h) {
   return (h->d.jp % 2 == 0) && h->p_consistent && h->cn1_separable && h->split_ok;
 }
 
+// The chip-resident solve (les_sor_res.hip) applies: a uniform horizontal grid that fits the
+// chip's LDS and registers, mirror-consistent p halos, cn1 of the separable form, no residual
+// between iterations, and the form not set by hand.  Any parity of jp.  It is the faster form
+// wherever it fits (300x300x90: see the kernel's comment), so nothing is timed to choose it.
+bool chip_solve(les_handle* h, bool resid) {
+  return !resid && h->sp.uniform && h->p_consistent && h->cn1_separable && h->split_ok &&
+         !h->sor_form_set && h->cfg.nmaxp > 0 && res_ready(h);
+}
+
+int launch_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_pav) {
+  auto go = [&]() {
+    launch_sor_resident(h->st, h->d, grid_of(h), h->sp, ph, h->cfg.nmaxp, h->sc, sub_rhsav, sub_pav,
+                        h->ra[0], h->ra[1], h->rplan, h->rbuf, h->res_wait);
+    return check_launch(h);
+  };
+  if (h->capturing) {
+    h->graph_chip = true;
+    return go();
+  }
+  return res_in_turn(h, h->st, go);
+}
+
 // press.f95:87-115 on the Fortran arrays: colour sweep, boundp1 per colour, boundp2 per
 // iteration (exact for any input state)
 int enqueue_sor_inplace(les_handle* h) {
@@ -927,6 +1028,7 @@ int enqueue_sor_split_loop(les_handle* h, bool allow_exit = true, const Physics*
   const Physics ph = phys ? *phys : h->ph;
   if (reset) launch_sor_reset(h->st, h->sc);
   const bool resid = allow_exit && h->ph.pjuge > 0.0f;
+  if (chip_solve(h, resid)) return launch_chip_solve(h, ph, 0, 0);
   int l0 = 1;
   if (!resid && h->iter_shape.tj > 0 && sor_iter_supported(d, h->sp)) {
     const SorPair fwd{{h->sp.p[0], h->sp.p[1]}, {h->palt[0], h->palt[1]}};
@@ -948,7 +1050,7 @@ int enqueue_sor_split_loop(les_handle* h, bool allow_exit = true, const Physics*
 int enqueue_sor_solve(les_handle* h) {
   STAGE_BEGIN(h);
   int r;
-  if (use_split(h)) {
+  if (use_split(h) || chip_solve(h, h->ph.pjuge > 0.0f)) {
     launch_split_scatter(h->st, d, F, h->sp, h->sc, 0);
     if ((r = enqueue_sor_split_loop(h))) return r;
     launch_split_gather_adj(h->st, d, F, h->sp, h->sc, 0);
@@ -1063,9 +1165,11 @@ int enqueue_press_mixed(les_handle* h) {
 
 // The resident split solve applies: fused iterations in pairs, no residual, FP32 with exact
 // sums, p and rhs not handed out by address.
-bool resident_applies(const les_handle* h) {
-  return h->resident_ok && use_split(h) && !(h->ph.pjuge > 0.0f) && h->iter_shape.tj > 0 &&
-         sor_iter_supported(h->d, h->sp) && h->cfg.nmaxp >= 2 && h->cfg.nmaxp % 2 == 0;
+bool resident_applies(les_handle* h) {
+  if (!h->resident_ok || h->ph.pjuge > 0.0f) return false;
+  if (chip_solve(h, false)) return true;
+  return use_split(h) && h->iter_shape.tj > 0 && sor_iter_supported(h->d, h->sp) &&
+         h->cfg.nmaxp >= 2 && h->cfg.nmaxp % 2 == 0;
 }
 
 // press.f95:49-146 on the resident split copy.  The split copy of p carries over from the last
@@ -1087,11 +1191,16 @@ int enqueue_press_resident(les_handle* h) {
                       carry ? 1 : 0};
   const SorPair fwd{{h->sp.p[0], h->sp.p[1]}, {h->palt[0], h->palt[1]}, {nullptr, nullptr}, 0};
   const SorPair back{{h->palt[0], h->palt[1]}, {h->sp.p[0], h->sp.p[1]}, {nullptr, nullptr}, 0};
-  launch_sor_iter(h->st, d, g, h->sp, h->ph, first, h->sc, h->iter_shape, 1);
-  launch_sor_iter(h->st, d, g, sra, h->ph, back, h->sc, h->iter_shape);
-  for (int l = 3; l + 1 <= h->cfg.nmaxp; l += 2) {
-    launch_sor_iter(h->st, d, g, sra, h->ph, fwd, h->sc, h->iter_shape);
+  if (chip_solve(h, false)) {
+    const int r = launch_chip_solve(h, h->ph, 1, carry ? 1 : 0);
+    if (r) return r;
+  } else {
+    launch_sor_iter(h->st, d, g, h->sp, h->ph, first, h->sc, h->iter_shape, 1);
     launch_sor_iter(h->st, d, g, sra, h->ph, back, h->sc, h->iter_shape);
+    for (int l = 3; l + 1 <= h->cfg.nmaxp; l += 2) {
+      launch_sor_iter(h->st, d, g, sra, h->ph, fwd, h->sc, h->iter_shape);
+      launch_sor_iter(h->st, d, g, sra, h->ph, back, h->sc, h->iter_shape);
+    }
   }
   launch_pav_split(h->st, d, g, h->sp, h->rb, h->sc);
   launch_split_gather_adj(h->st, d, F, h->sp, h->sc, 1, 1);  // p - pav, halos; pav_carry
@@ -1110,7 +1219,7 @@ int enqueue_press(les_handle* h) {
   h->rhs_stale = false;  // F.rhs is written below
   int r;
   enqueue_rhs_rhsav(h, d, g, F);
-  if (use_split(h)) {
+  if (use_split(h) || chip_solve(h, h->ph.pjuge > 0.0f)) {
     launch_split_scatter(h->st, d, F, h->sp, h->sc, 1);  // rhs -= rhsav on the way
     if ((r = enqueue_sor_split_loop(h, true, nullptr, false))) return r;
     if (seq_sums(h))
@@ -1267,8 +1376,12 @@ int ensure_graph(les_handle* h) {
   if (h->graph) hipGraphDestroy(h->graph);
   h->gexec = nullptr;
   h->graph = nullptr;
+  (void)res_ready(h);  // no allocation inside the capture
+  h->graph_chip = false;
   HIPCHK(h, hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal));
+  h->capturing = true;
   int r = enqueue_step(h, 2);
+  h->capturing = false;
   hipGraph_t gr = nullptr;
   hipError_t e = hipStreamEndCapture(h->st, &gr);
   if (r) {
@@ -1281,6 +1394,12 @@ int ensure_graph(les_handle* h) {
   h->graph_valid = true;
   h->graph_resident = h->sp_p_current;  // set by the captured step iff it is resident
   return LES_OK;
+}
+
+// one replay of the captured step (in its turn, when it runs the chip-resident solve)
+hipError_t replay_step(les_handle* h) {
+  if (!h->graph_chip) return hipGraphLaunch(h->gexec, h->st);
+  return res_in_turn(h, h->st, [&]() { return hipGraphLaunch(h->gexec, h->st); });
 }
 
 // the host-side state a replay of the captured step leaves
@@ -1300,7 +1419,7 @@ extern "C" int les_run(les_handle* h, int n0, int nsteps) {
   if (r) return r;
   if (nsteps == 0) return LES_OK;
   if ((r = ensure_graph(h))) return r;
-  for (int s = 0; s < nsteps; ++s) HIPCHK(h, hipGraphLaunch(h->gexec, h->st));
+  for (int s = 0; s < nsteps; ++s) HIPCHK(h, replay_step(h));
   after_replays(h);
   return LES_OK;
 }
@@ -1622,7 +1741,7 @@ extern "C" int les_ensemble_run(les_ensemble* e, int n0, int nsteps) {
     for (int q = 0; q < nm; ++q) {
       les_handle* h = e->m[q];
       if (s < nsteps - left[q]) continue;  // this member ran its first steps eagerly
-      HIPCHK(h, hipGraphLaunch(h->gexec, h->st));
+      HIPCHK(h, replay_step(h));
     }
   for (int q = 0; q < nm; ++q)
     if (left[q] > 0) after_replays(e->m[q]);
@@ -1807,7 +1926,7 @@ extern "C" int les_time_kernel(les_handle* h, int which, int reps, float* avg_ms
       case LES_KERNEL_CALC_SM: launch_calc_sm(h->st, d, g, F, h->ph, 0, h->shp_sm); break;
       case LES_KERNEL_RHS: launch_rhs(h->st, d, g, F, h->ph, h->rb, h->sc); break;
       case LES_KERNEL_VELNW: launch_velnw_inflow(h->st, d, g, F, h->ph, 1, 2, h->shp_velnw); break;
-      case LES_KERNEL_STEP: HIPCHK(h, hipGraphLaunch(h->gexec, h->st)); break;
+      case LES_KERNEL_STEP: HIPCHK(h, replay_step(h)); break;
       case LES_KERNEL_SOR_ITER: {
         if (!sor_iter_supported(d, h->sp)) {
           hipEventDestroy(e0);
@@ -1835,6 +1954,15 @@ extern "C" int les_time_kernel(les_handle* h, int which, int reps, float* avg_ms
   return check_launch(h);
 }
 
+// Not part of the ABI: how long (100 MHz ticks) the chip-resident solve's workgroups wait for each
+// other before the queue form; negative: the queue form at once.  For the test of that form.
+extern "C" int les_internal_sor_wait(les_handle* h, long ticks) {
+  if (!h) return LES_E_INVALID;
+  h->res_wait = ticks;
+  h->graph_valid = false;
+  return LES_OK;
+}
+
 extern "C" int les_set_sor_tile(les_handle* h, int tile_j, int tile_k) {
   if (!h) return LES_E_INVALID;
   if (tile_j == 0) {
@@ -1847,6 +1975,7 @@ extern "C" int les_set_sor_tile(les_handle* h, int tile_j, int tile_k) {
       return fail(h, LES_E_STATE, "set_sor_tile: the fused SOR iteration does not apply to this grid");
     h->iter_shape = SorIterShape{tile_j, tile_k};
   }
+  h->sor_form_set = true;
   h->graph_valid = false;
   return LES_OK;
 }

@@ -1,0 +1,45 @@
+// The chip-resident SOR solve (les_sor_res.hip): plan, buffers and launch.
+#pragma once
+#include "les_kernels.h"
+
+namespace les {
+
+constexpr int RES_NT = 512;     // threads per workgroup
+constexpr int RES_TKMAX = 10;   // most levels per thread
+constexpr int RES_TK_KS = 7;    // ... with more than one level block per workgroup (LDS)
+constexpr int RES_KWMAX = 128;  // most levels per workgroup
+constexpr int RES_JS = 64;      // most groups per row (ip <= 512)
+
+// How the domain is cut: njt x nkt workgroups of rj rows of j and ks * tk levels; ks level
+// blocks of tk levels each, one thread per (group of four entries, row, level block).
+struct ResPlan {
+  int tk = 0;  // 0: the grid does not fit
+  int ks = 0, rj = 0, njt = 0, nkt = 0;
+  __host__ __device__ int nwg() const { return njt * nkt; }
+};
+
+constexpr long RES_WAIT_TICKS = 30000;  // 0.3 ms of the 100 MHz clock
+
+struct ResCtl;  // device control block (les_sor_res.hip)
+
+// Face slots and control block of one handle (res_alloc / res_free)
+struct ResBuf {
+  unsigned long long* kslot = nullptr;
+  unsigned long long* jslot = nullptr;
+  float* seam = nullptr;
+  ResCtl* ctl = nullptr;
+};
+
+ResPlan res_plan(Dims d, int nr, int ncu);
+hipError_t res_alloc(Dims d, int nr, const ResPlan& pl, hipStream_t st, ResBuf& b);
+void res_free(ResBuf& b);
+// nmaxp SOR iterations (press.f95:87-115 without early exit) on the split copy sp.p / sp.r in
+// place.  sub_rhsav: sp.r holds the raw rhs; rhsav is taken off every value read and the result
+// written to rout.  sub_pav: DevScalars::pav_carry is taken off every p value read.  wait_ticks
+// (100 MHz): how long the workgroups wait for each other to be resident before the solve falls
+// back to the queue form; negative: the queue form at once.
+void launch_sor_resident(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Physics ph, int nmaxp,
+                         const DevScalars* sc, int sub_rhsav, int sub_pav, float* rout0,
+                         float* rout1, const ResPlan& pl, const ResBuf& b, long wait_ticks);
+
+}  // namespace les

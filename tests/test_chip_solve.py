@@ -1,0 +1,83 @@
+"""The SOR solve held on the chip (one launch, les_sor_res.hip) against the colour sweeps, bit for
+bit: cuts with one and several workgroups along j and k, partial top level blocks and last rows,
+colour rows with padding, odd jp (the periodic seam joins cells of one colour), the largest
+number of levels per thread; the queue form that serves it when its workgroups cannot all be
+resident; and two handles taking turns on one device."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import common
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("p", "u", "v", "w", "rhs")
+
+
+def _handle(dims, nmaxp, sweeps, dx=4.0):
+    from les_halo_amd import LES, inputs
+    L = LES(*dims, **common.REF_PHYS, omega=1.5, pjuge=0.0, nmaxp=nmaxp)
+    L.load_case(inputs.make_case(*dims, seed=5, hmax=20.0, dx=dx))
+    L.ifdata()
+    if sweeps:
+        L.set_sor_tile(0)
+    return L
+
+
+def _same(a, b, names=FIELDS):
+    for nm in names:
+        x, y = a.download(nm), b.download(nm)
+        assert common.bits_equal(x, y), common.mismatch_report(x, y, nm)
+    assert np.abs(a.download("p")).max() > 0
+
+
+# 1 workgroup; level blocks in one workgroup, the last partial; several along k; along j and k
+# with a partial top block; odd jp in one tile and in several; ip > 320; 9 levels a thread
+GRIDS = [(16, 12, 10), (31, 18, 17), (48, 48, 32), (150, 44, 61), (35, 27, 19), (20, 5, 7),
+         (147, 133, 61), (512, 100, 20), (300, 300, 90)]
+
+
+@pytest.mark.parametrize("dims", GRIDS)
+@pytest.mark.parametrize("dx", [4.0, 5.0])
+def test_chip_solve_equals_colour_sweeps(dims, dx):
+    print(dims, dx, flush=True)
+    a, b = _handle(dims, 7, False, dx), _handle(dims, 7, True, dx)
+    a.run(1, 4)   # eager first step, then graph replays that carry the split copy
+    b.run(1, 4)
+    _same(a, b)
+    a.press_sor_solve()  # scatter, solve, gather
+    b.press_sor_solve()
+    _same(a, b, ("p",))
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("dims", [(32, 24, 16), (96, 96, 20), (35, 27, 19)])
+def test_queue_form_equals_colour_sweeps(dims):
+    from les_halo_amd._lib import lib
+    print(dims, flush=True)
+    a, b = _handle(dims, 6, False), _handle(dims, 6, True)
+    assert lib().les_internal_sor_wait(a.h, ctypes.c_long(-1)) == 0
+    a.run(1, 4)
+    b.run(1, 4)
+    _same(a, b)
+    assert lib().les_internal_sor_wait(a.h, ctypes.c_long(30000)) == 0
+    a.run(5, 2)   # back to the resident form on the same buffers
+    b.run(5, 2)
+    _same(a, b)
+    a.close()
+    b.close()
+
+
+def test_two_handles_take_turns():
+    dims = (150, 150, 30)
+    hs = [_handle(dims, 10, False) for _ in range(2)] + [_handle(dims, 10, True)]
+    for n in range(1, 9, 2):  # enqueued without waiting in between
+        for h in hs[:2]:
+            h.run(n, 2)
+    hs[2].run(1, 8)
+    for h in hs[:2]:
+        _same(h, hs[2])
+    for h in hs:
+        h.close()
