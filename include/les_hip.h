@@ -120,8 +120,9 @@ typedef struct les_config {
   float refine_omega; /* LES_PREC_MIXED: relaxation of the correction solves' SOR sweeps; 0 =
                          omega (SOR corrections) or 1 (the CG preconditioner) */
   int refine_solver;  /* LES_PREC_MIXED: 0 = each correction by nmaxp SOR iterations from zero;
-                         1 = by nmaxp conjugate-gradient iterations preconditioned by symmetric
-                         red-black Gauss-Seidel (the FP32 colour sweeps), FP64 inner products */
+                         1 = by conjugate gradients (at most 20 nmaxp iterations) preconditioned
+                         by symmetric red-black Gauss-Seidel, on a uniform horizontal grid with
+                         a multigrid V-cycle inside it, FP64 inner products */
   int sum_order;      /* LES_SUM_EXACT or LES_SUM_REFERENCE (FP32 single-domain handles only) */
 } les_config;
 

@@ -15,6 +15,7 @@
 
 #include "../../include/les_hip.h"
 #include "les_kernels.h"
+#include "les_mg.h"
 #include "les_mixed.h"
 #include "les_sor_res.h"
 
@@ -47,6 +48,8 @@ struct les_handle {
   Mixed mx{};
   double* mx_mem = nullptr;
   float* cg_mem = nullptr;  // mixed precision: the conjugate-gradient vectors
+  MgPlan mg;                // ... and their preconditioner's coarse grids
+  bool mg_current = false;  // they are of the grid now loaded
   // second iterate of the fused SOR iteration (ping-pong with sp.p) and its workgroup tile
   float* palt[2] = {nullptr, nullptr};
   SorIterShape iter_shape{0, 0};  // tj == 0: two colour sweeps per iteration (untuned default)
@@ -629,6 +632,7 @@ extern "C" int les_destroy(les_handle* h) {
   if (h->split_mem) hipFree(h->split_mem);
   if (h->mx_mem) hipFree(h->mx_mem);
   if (h->cg_mem) hipFree(h->cg_mem);
+  mg_release(h->mg);
   if (h->ave_mem) hipFree(h->ave_mem);
   if (h->seq_mem) hipFree(h->seq_mem);
   if (h->st) hipStreamDestroy(h->st);
@@ -663,7 +667,10 @@ extern "C" int les_upload(les_handle* h, int field, const float* host) {
   }
   HIPCHK(h, hipStreamSynchronize(h->st));
   HIPCHK(h, hipMemcpy(h->fld[field], host, n * sizeof(float), hipMemcpyHostToDevice));
-  if (!h->hgrid[field].empty()) std::memcpy(h->hgrid[field].data(), host, n * sizeof(float));
+  if (!h->hgrid[field].empty()) {
+    std::memcpy(h->hgrid[field].data(), host, n * sizeof(float));
+    h->mg_current = false;
+  }
   if (is_mask(field)) {
     // rebuild the interior bit mask from the four device masks
     std::vector<float> hm[4];
@@ -1150,7 +1157,20 @@ int enqueue_press_mixed(les_handle* h) {
       // preconditioner relaxation: refine_omega, else 1 (symmetric Gauss-Seidel; at 600x600x90
       // 1420 iterations per step against 1600 for 1.5 and 2330 for 1.8)
       const float om = h->cfg.refine_omega > 0.0f ? h->cfg.refine_omega : 1.0f;
-      launch_mx_cg(h->st, d, g, h->sp, h->mx, 20 * h->cfg.nmaxp, om, stop);
+      // The coarse grids want one horizontal spacing and plain Gauss-Seidel (om 1, the default):
+      // 300x300x90 to 1e-7: see les_mg.hip.  Without memory for them: the pass alone.
+      const MgPlan* mg = nullptr;
+      if (h->sp.uniform && om == 1.0f) {
+        if (!h->mg_current) {
+          HIPCHK(h, hipStreamSynchronize(h->st));
+          if (mg_setup(d, h->hgrid[LES_CN2L][0], h->hgrid[LES_CN3L][0], h->hgrid[LES_CN4L],
+                       h->hgrid[LES_CN4S], h->mg) != hipSuccess)
+            (void)hipGetLastError();
+          h->mg_current = true;
+        }
+        if (h->mg.nl > 0) mg = &h->mg;
+      }
+      launch_mx_cg(h->st, d, g, h->sp, h->mx, 20 * h->cfg.nmaxp, om, stop, mg);
     }
     if (h->cfg.refine_solver != 1 && (r = enqueue_sor_split_loop(h, false, &ph_corr))) return r;
     launch_mx_accumulate(h->st, d, h->sp, h->mx);

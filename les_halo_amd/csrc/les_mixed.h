@@ -34,9 +34,11 @@ void launch_mx_accumulate(hipStream_t st, Dims d, SplitSOR sp, Mixed mx);
 // the correction solve as conjugate gradients on -L e = -r (sp.r: r, sp.p: e from zero),
 // preconditioned by symmetric red-black SOR with relaxation om; at most iters iterations,
 // stopping on the device once the preconditioned residual norm squared falls to stop times its
-// start value
+// start value; mg: with a coarse-grid correction inside that pass (om = 1).  Waits for the device
+// now and then to see whether the iterations have stopped.
+struct MgPlan;
 void launch_mx_cg(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Mixed mx, int iters, float om,
-                  double stop);
+                  double stop, const MgPlan* mg);
 void launch_mx_pav_gather(hipStream_t st, Dims d, Grid1D g, Fields F, SplitSOR sp, Mixed mx,
                           DevScalars* sc);
 

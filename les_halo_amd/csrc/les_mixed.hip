@@ -17,7 +17,7 @@
 // In exact arithmetic SOR from p on rhs equals p plus SOR from 0 on rhs - L p, so each pass
 // continues the reference iteration while FP64 carries the accumulated solution.  All state is
 // in the colour-split layout of les_sor.hip (interior cells, colour (i+j+k)&1).
-#include "les_mixed.h"
+#include "les_mg.h"
 
 #include <algorithm>
 #include <utility>
@@ -489,6 +489,9 @@ __global__ __launch_bounds__(256) void k_cg_apply(Dims d, Grid1D g, SplitSOR sp,
 //           iteration's e += alpha dnew, rr += alpha q on both colours (q = A dnew = -L dnew);
 //   PASS 1: colour 1 from the colour-0 neighbours, z_1 = om (2 - om) gs;
 //   PASS 2: colour 0, z_0 = (1 - om) z_0 + om gs, and block partials of <rr, z>.
+// Around a coarse-grid correction (om = 1; les_mg.hip) pass 1 runs before and after it, and
+//   PASS 3: colour 0's residual after passes 0 and 1, sum c_nb z_nb, into mx.q[0] (colour 1's is
+//           zero, and its correction would be overwritten by the second pass 1).
 template <int PASS, bool UPDATE>
 __global__ __launch_bounds__(256) void k_cg_sgs(Dims d, Grid1D g, SplitSOR sp, Mixed mx, float om,
                                                 CgDir dd, int nthreads) {
@@ -563,6 +566,15 @@ __global__ __launch_bounds__(256) void k_cg_sgs(Dims d, Grid1D g, SplitSOR sp, M
         t += c4s * zm[q];
         s[q] = t;
       }
+    }
+    if constexpr (PASS == 3) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (f + 1 + 2 * (4 * grp + q) > d.ip) s[q] = 0.0f;
+      if (it.ok) st4(mx.q[C] + b, s);
+      copy4(zm, zc);
+      copy4(zc, zp);
+      continue;
     }
     float zo[4] = {0, 0, 0, 0};
     if constexpr (PASS == 2) unpack(ld4(mx.z[C] + b), zo);
@@ -673,7 +685,7 @@ __global__ __launch_bounds__(256) void k_cg_project(Dims d, SplitSOR sp, Mixed m
 }
 
 void launch_mx_cg(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Mixed mx, int iters, float om,
-                  double stop) {
+                  double stop, const MgPlan* mg) {
   const dim3 grid = mx_grid(d), blk(MX_BX, MX_BY);
   CgDir dd{{mx.dir[0], mx.dir[1]}, {mx.dir2[0], mx.dir2[1]}};
   // four entries of a colour row over CG_KC levels per thread
@@ -686,6 +698,11 @@ void launch_mx_cg(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Mixed mx, int i
     else
       hipLaunchKernelGGL((k_cg_sgs<0, false>), cg, cb, 0, st, d, g, sp, mx, om, dd, nt);
     hipLaunchKernelGGL((k_cg_sgs<1, false>), cg, cb, 0, st, d, g, sp, mx, om, dd, nt);
+    if (mg) {
+      hipLaunchKernelGGL((k_cg_sgs<3, false>), cg, cb, 0, st, d, g, sp, mx, om, dd, nt);
+      launch_mg_correct(st, d, sp, mx, *mg);
+      hipLaunchKernelGGL((k_cg_sgs<1, false>), cg, cb, 0, st, d, g, sp, mx, om, dd, nt);
+    }
     hipLaunchKernelGGL((k_cg_sgs<2, false>), cg, cb, 0, st, d, g, sp, mx, om, dd, nt);
   };
   hipLaunchKernelGGL(k_cg_reset, dim3(1), dim3(64), 0, st, mx);
@@ -694,6 +711,9 @@ void launch_mx_cg(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Mixed mx, int i
   hipLaunchKernelGGL(k_cg_project, grid, blk, 0, st, d, sp, mx);
   precondition(false);
   hipLaunchKernelGGL(k_cg_scalar, dim3(1), dim3(256), 0, st, mx, 0, stop, nwg);
+  // How many iterations are enqueued before the host looks whether they have stopped: an
+  // iteration past the stop still costs its launches.
+  const int batch = mg ? 4 : 64;
   for (int it = 0; it < iters; ++it) {
     // dnew = z + beta dold into the other buffer; q = A dnew; alpha
     if (it == 0)
@@ -705,6 +725,13 @@ void launch_mx_cg(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Mixed mx, int i
     hipLaunchKernelGGL(k_cg_scalar, dim3(1), dim3(256), 0, st, mx, 2, stop, nwg);
     std::swap(dd.old_[0], dd.new_[0]);
     std::swap(dd.old_[1], dd.new_[1]);
+    if (it % batch == batch - 1) {
+      double stopped = 0.0;
+      if (hipMemcpyAsync(&stopped, mx.cg + 4, sizeof stopped, hipMemcpyDeviceToHost, st) != hipSuccess ||
+          hipStreamSynchronize(st) != hipSuccess)
+        return;  // the caller's next call reports it
+      if (stopped != 0.0) break;
+    }
   }
 }
 
