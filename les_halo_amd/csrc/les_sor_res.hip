@@ -45,7 +45,7 @@
 // 9 levels): 2.0 us computing (77 vector instructions a group of four cells, two wavefronts per
 // SIMD), 0.9 us more with k faces only, 5.0 us with both; memory is read once and written once
 // per solve.  50 iterations, measured with the scatter and gather of p around them: 300x300x90
-// 592 us against 50 x 20.5 us for k_sor_iter; 150x150x90 325 against 50 x 11.7; 32x24x16 133
+// 592 us against 50 x 20.5 us for k_sor_iter; 150x150x90 303 against 50 x 11.7; 32x24x16 133
 // against 50 x 8.3; 147x133x61 (odd jp) about 320 against 100 x (9.2 + 4.9) + 50 x 4.6 in place.
 #include <algorithm>
 
@@ -635,10 +635,11 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
 
 }  // namespace
 
-// The cut with the least estimated time per sweep, from the times measured for a sweep's parts:
-// 0.06 us a level plus 0.07 us for each wavefront of the busiest SIMD (0.25 us at one level, 2.0 us
-// at nine levels and two wavefronts, without faces), 0.9 us where there are k faces (their words
-// go out and come back within the sweep), 1.0 us where there are j faces (the same, and a barrier).
+// The cut with the least estimated time per sweep in us, fitted to the times of 40 cuts of
+// 150x150x90 and 96x96x60 and of smaller grids: per level 0.25 plus 0.045 for each wavefront of the
+// busiest SIMD; 0.9 for any faces, 0.28 per 1000 words of the k faces, 0.25 and 0.1 per 1000 words
+// for j faces, 0.15 where the XCDs' shares cut through a row of workgroups along k.  It prefers cuts about as high as they are long: 96x96x60 in 8 levels x 5 rows takes 1.7 us a sweep, in 1 x 32 2.3; 150x150x90
+// in 6 x 13 2.6, in 3 x 25 2.9.
 ResPlan res_plan(Dims d, int nr, int ncu) {
   ncu = std::min(ncu, RES_WGMAX);
   ResPlan best;
@@ -654,9 +655,11 @@ ResPlan res_plan(Dims d, int nr, int ncu) {
         const int nkt = (d.kp + ks * tk - 1) / (ks * tk);
         if ((long)njt * nkt > ncu || 4 * ng * ks * tk > res_jn(tk) * RES_NT) continue;
         const int waves = (rj * ks * ng + 63) / 64;
-        const double cost = tk * (0.06 + 0.07 * ((waves + 3) / 4) + (ks > 1 ? 0.02 : 0.0)) +
-                            (nkt > 1 ? 0.9 : 0.0) + (njt > 1 || d.jp % 2 ? 1.0 : 0.0) +
-                            1e-4 * njt * nkt;
+        const bool fk = nkt > 1, fj = njt > 1 || d.jp % 2;
+        const double cost = tk * (0.25 + 0.045 * ((waves + 3) / 4)) + (fk || fj ? 0.9 : 0.0) +
+                            (fk ? 0.28e-3 * (8 * rj * ng) : 0.0) +
+                            (fj ? 0.25 + 0.1e-3 * (8 * ks * tk * ng) : 0.0) +
+                            (fj && njt % 8 ? 0.15 : 0.0) + 1e-4 * njt * nkt;
         if (best.tk == 0 || cost < best_cost) {
           best_cost = cost;
           best.tk = tk;
