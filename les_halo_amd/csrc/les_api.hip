@@ -986,18 +986,19 @@ bool use_split(const les_handle* h) {
 }
 
 // The chip-resident solve (les_sor_res.hip) applies: a uniform horizontal grid that fits the
-// chip's LDS and registers, mirror-consistent p halos, cn1 of the separable form, no residual
-// between iterations, and the form not set by hand.  Any parity of jp.  It is the faster form
-// wherever it fits (300x300x90: see the kernel's comment), so nothing is timed to choose it.
+// chip's LDS and registers, mirror-consistent p halos, cn1 of the separable form, no residual in
+// the reference's order of terms, and the form not set by hand.  Any parity of jp.  It is the
+// faster form wherever it fits (300x300x90: see the kernel's comment), so nothing is timed to
+// choose it.
 bool chip_solve(les_handle* h, bool resid) {
-  return !resid && h->sp.uniform && h->p_consistent && h->cn1_separable && h->split_ok &&
+  return !(resid && seq_sums(h)) && h->sp.uniform && h->p_consistent && h->cn1_separable && h->split_ok &&
          !h->sor_form_set && h->cfg.nmaxp > 0 && res_ready(h);
 }
 
-int launch_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_pav) {
+int launch_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_pav, bool resid) {
   auto go = [&]() {
     launch_sor_resident(h->st, h->d, grid_of(h), h->sp, ph, h->cfg.nmaxp, h->sc, sub_rhsav, sub_pav,
-                        h->ra[0], h->ra[1], h->rplan, h->rbuf, h->res_wait);
+                        h->ra[0], h->ra[1], resid ? h->rb.slots : nullptr, h->rplan, h->rbuf, h->res_wait);
     return check_launch(h);
   };
   if (h->capturing) {
@@ -1035,7 +1036,7 @@ int enqueue_sor_split_loop(les_handle* h, bool allow_exit = true, const Physics*
   const Physics ph = phys ? *phys : h->ph;
   if (reset) launch_sor_reset(h->st, h->sc);
   const bool resid = allow_exit && h->ph.pjuge > 0.0f;
-  if (chip_solve(h, resid)) return launch_chip_solve(h, ph, 0, 0);
+  if (chip_solve(h, resid)) return launch_chip_solve(h, ph, 0, 0, resid);
   int l0 = 1;
   if (!resid && h->iter_shape.tj > 0 && sor_iter_supported(d, h->sp)) {
     const SorPair fwd{{h->sp.p[0], h->sp.p[1]}, {h->palt[0], h->palt[1]}};
@@ -1183,12 +1184,13 @@ int enqueue_press_mixed(les_handle* h) {
   return check_launch(h);
 }
 
-// The resident split solve applies: fused iterations in pairs, no residual, FP32 with exact
-// sums, p and rhs not handed out by address.
+// The resident split solve applies: the chip-resident form, or fused iterations in pairs without
+// a residual; FP32 with exact sums, p and rhs not handed out by address.
 bool resident_applies(les_handle* h) {
-  if (!h->resident_ok || h->ph.pjuge > 0.0f) return false;
-  if (chip_solve(h, false)) return true;
-  return use_split(h) && h->iter_shape.tj > 0 && sor_iter_supported(h->d, h->sp) &&
+  const bool resid = h->ph.pjuge > 0.0f;
+  if (!h->resident_ok) return false;
+  if (chip_solve(h, resid)) return true;
+  return !resid && use_split(h) && h->iter_shape.tj > 0 && sor_iter_supported(h->d, h->sp) &&
          h->cfg.nmaxp >= 2 && h->cfg.nmaxp % 2 == 0;
 }
 
@@ -1211,8 +1213,9 @@ int enqueue_press_resident(les_handle* h) {
                       carry ? 1 : 0};
   const SorPair fwd{{h->sp.p[0], h->sp.p[1]}, {h->palt[0], h->palt[1]}, {nullptr, nullptr}, 0};
   const SorPair back{{h->palt[0], h->palt[1]}, {h->sp.p[0], h->sp.p[1]}, {nullptr, nullptr}, 0};
-  if (chip_solve(h, false)) {
-    const int r = launch_chip_solve(h, h->ph, 1, carry ? 1 : 0);
+  const bool resid = h->ph.pjuge > 0.0f;
+  if (chip_solve(h, resid)) {
+    const int r = launch_chip_solve(h, h->ph, 1, carry ? 1 : 0, resid);
     if (r) return r;
   } else {
     launch_sor_iter(h->st, d, g, h->sp, h->ph, first, h->sc, h->iter_shape, 1);

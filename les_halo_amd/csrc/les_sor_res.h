@@ -33,13 +33,14 @@ struct ResBuf {
 ResPlan res_plan(Dims d, int nr, int ncu);
 hipError_t res_alloc(Dims d, int nr, const ResPlan& pl, hipStream_t st, ResBuf& b);
 void res_free(ResBuf& b);
-// nmaxp SOR iterations (press.f95:87-115 without early exit) on the split copy sp.p / sp.r in
-// place.  sub_rhsav: sp.r holds the raw rhs; rhsav is taken off every value read and the result
-// written to rout.  sub_pav: DevScalars::pav_carry is taken off every p value read.  wait_ticks
-// (100 MHz): how long the workgroups wait for each other to be resident before the solve falls
-// back to the queue form; negative: the queue form at once.
+// nmaxp SOR iterations (press.f95:87-115) on the split copy sp.p / sp.r in place.  sub_rhsav: sp.r
+// holds the raw rhs; rhsav is taken off every value read and the result written to rout.
+// sub_pav: DevScalars::pav_carry is taken off every p value read.  resid_slots (RedBuf::slots, zero):
+// with the residual of every iteration (DevScalars::sor, sor_iters) and the early exit; null:
+// without.  wait_ticks (100 MHz): how long the workgroups wait for each other to be resident
+// before the solve falls back to the queue form; negative: the queue form at once.
 void launch_sor_resident(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Physics ph, int nmaxp,
-                         const DevScalars* sc, int sub_rhsav, int sub_pav, float* rout0,
-                         float* rout1, const ResPlan& pl, const ResBuf& b, long wait_ticks);
+                         DevScalars* sc, int sub_rhsav, int sub_pav, float* rout0, float* rout1,
+                         int64_t* resid_slots, const ResPlan& pl, const ResBuf& b, long wait_ticks);
 
 }  // namespace les

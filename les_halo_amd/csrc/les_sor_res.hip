@@ -56,6 +56,8 @@ namespace les {
 constexpr int RES_WGMAX = 1024;  // (no device has that many CUs)
 struct ResCtl {
   unsigned arrive, state, done, base, ticket, tasks;
+  // the residual: workgroups that have added theirs, iterations decided (times 2, plus 1: stop)
+  unsigned added, decided;
   unsigned xcd[RES_WGMAX];  // the XCD each workgroup of the launch is on
 };
 
@@ -77,9 +79,11 @@ struct ResArgs {
   SplitSOR sp;
   float omega;
   int nmaxp;
-  const DevScalars* sc;
+  DevScalars* sc;
   int sub_rhsav, sub_pav;
   float* rout[2];
+  float pjuge;
+  int64_t* slots;  // exact-sum slots of the residual (RedBuf::slots), zero between uses
   ResPlan pl;
   u64 *kslot, *jslot;
   float* seam;
@@ -177,6 +181,101 @@ __device__ __forceinline__ void lds_only_barrier() {
   __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// Exact sum of the residual's terms reltmp**2 (never negative) of one thread and iteration: a term
+// m 2^(s-149) goes, shifted to its limb's origin, into one of three 64-bit sums for three limbs
+// next to each other (at most 2 * 4 * RES_TKMAX terms below 2^56 each: no overflow), the rare
+// others straight into the workgroup's limbs.  The integers added are those of ThreadAcc.
+struct SquareAcc {
+  u64 a0 = 0, a1 = 0, a2 = 0;
+  int base = -1;
+  __device__ __forceinline__ void add(float x, u64* lds) {
+    const unsigned b = __float_as_uint(x), e = b >> 23;  // sign 0
+    unsigned m = b & 0x7fffffu;
+    if (e) m |= 0x800000u;
+    if (e >= 0xffu) m = 0u;  // inf and nan are not summed
+    const int s = max((int)e, 1) - 1;
+    const u64 v = (u64)m << (s & 31);
+    if (base < 0 && m) base = min(max((s >> 5) - 1, 0), NLIMB - 4);
+    const int d = (s >> 5) - base;
+    a0 += d == 0 ? v : 0;
+    a1 += d == 1 ? v : 0;
+    a2 += d == 2 ? v : 0;
+    if ((d < 0 || d > 2) && m) {
+      atomicAdd(&lds[s >> 5], v & 0xffffffffull);
+      atomicAdd(&lds[(s >> 5) + 1], v >> 32);
+    }
+  }
+  // every lane of the wavefront together
+  __device__ __forceinline__ void flush(u64* lds) {
+    ThreadAcc t;
+    t.base = base;
+    t.r0 = (int64_t)(a0 & 0xffffffffull);
+    t.r1 = (int64_t)((a0 >> 32) + (a1 & 0xffffffffull));
+    t.r2 = (int64_t)((a1 >> 32) + (a2 & 0xffffffffull));
+    t.r3 = (int64_t)(a2 >> 32);
+    t.flush(lds);
+    a0 = a1 = a2 = 0;
+    base = -1;
+  }
+};
+
+// this wavefront's own stores and atomics have reached memory.  What the workgroups exchange about
+// the residual is read and written by agent-scope atomics alone, so their order is all that is
+// needed; a fence would write the L2 back (the faces kept within an XCD) at every iteration.
+__device__ __forceinline__ void mem_done() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// One thread: the residual from the limbs (press.f95:97), the iteration's count and the early
+// exit (press.f95:114); tells the other workgroups.  Agent scope: another iteration's decision may
+// be taken on another XCD.
+__device__ inline unsigned res_decide(const ResArgs& a, const int64_t* limbs, unsigned it) {
+  const float s = limbs_to_float(limbs);
+  const bool stop = s < a.pjuge;
+  agent_store(&a.sc->sor, s);
+  agent_store(&a.sc->sor_iters, (int)it);
+  if (stop) agent_store(&a.sc->sor_done, 1);
+  const unsigned dec = 2u * it + (stop ? 1u : 0u);
+  mem_done();
+  agent_store(&a.ctl->decided, dec);
+  mem_done();
+  return dec;
+}
+
+// The whole workgroup: adds its limbs (in LDS, cleared again) to the slots, and returns whether it
+// was the last of 'n' to do so; that one then has all limbs in 'limbs' and the slots are zero.
+__device__ inline bool res_add_limbs(const ResArgs& a, u64* lds, unsigned* counter, unsigned n,
+                                     int64_t* limbs, unsigned* flag) {
+  const int t = threadIdx.x;
+  __syncthreads();
+  u64* slots = reinterpret_cast<u64*>(a.slots);
+  if (t < NLIMB) {
+    if (lds[t]) atomicAdd(slots + (blockIdx.x % RED_SLOTS) * NLIMB + t, lds[t]);
+    lds[t] = 0;
+    mem_done();  // added before counted
+  }
+  __syncthreads();
+  if (t == 0)
+    *flag = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == n;
+  __syncthreads();
+  const bool last = *flag != 0u;
+  if (last) {
+    for (int q = t; q < RED_SLOTS * NLIMB; q += RES_NT) {
+      const u64 v = agent_load(slots + q);
+      if (v) {
+        atomicAdd(&lds[q % NLIMB], v);
+        agent_store(slots + q, (u64)0);
+      }
+    }
+    mem_done();  // cleared before anyone is told
+    __syncthreads();
+    if (t < NLIMB) {
+      limbs[t] = (int64_t)lds[t];
+      lds[t] = 0;
+    }
+  }
+  __syncthreads();
+  return last;
+}
+
 // The last workgroup to leave re-arms the control block for the next launch (stream order makes
 // it visible there).
 __device__ __forceinline__ void res_leave(const ResArgs& a) {
@@ -188,6 +287,8 @@ __device__ __forceinline__ void res_leave(const ResArgs& a) {
   agent_store(&a.ctl->arrive, 0u);
   agent_store(&a.ctl->ticket, 0u);
   agent_store(&a.ctl->tasks, 0u);
+  agent_store(&a.ctl->added, 0u);
+  agent_store(&a.ctl->decided, 0u);
   agent_store(&a.ctl->done, 0u);
   agent_store(&a.ctl->state, 0u);
 }
@@ -195,9 +296,14 @@ __device__ __forceinline__ void res_leave(const ResArgs& a) {
 // The same solve through the task queue, on the split copy in device memory.  Phases in order:
 // the rhsav / pav shifts, then per sweep (odd jp: a copy of the two seam rows of the colour,
 // the values before the sweep, and) the sweep; nb tasks of RES_NT groups per phase.  A task of
-// phase f starts when f * nb tasks have ended.
+// phase f starts when f * nb tasks have ended.  With the residual, the workgroup that adds the last
+// of an iteration's limbs decides before its task ends; after a stop the tasks left are void.
+template <bool RESID>
 __device__ void res_queue(const ResArgs& a) {
-  __shared__ unsigned sTask;
+  __shared__ unsigned sTask, sFlag;
+  __shared__ u64 sLimb[NLIMB];
+  __shared__ int64_t sSum[NLIMB];
+  if (RESID && threadIdx.x < NLIMB) sLimb[threadIdx.x] = 0;
   const Dims& d = a.d;
   const SplitSOR& sp = a.sp;
   const int ng = sp.nr / 4, pl = sp.nr * sp.nj;
@@ -215,7 +321,14 @@ __device__ void res_queue(const ResArgs& a) {
       sTask = n;
       if (n < nphase * nb) {
         const unsigned need = n / nb * nb;
-        while (agent_load(&a.ctl->tasks) < need) __builtin_amdgcn_s_sleep(4);
+        bool stop = false;  // (decided before the iteration's last task ends)
+        for (;;) {
+          const bool go = agent_load(&a.ctl->tasks) >= need;
+          if (RESID) stop = agent_load(&a.ctl->decided) & 1u;
+          if (go || stop) break;
+          __builtin_amdgcn_s_sleep(4);
+        }
+        if (stop) sTask = 0xffffffffu;
       }
     }
     __syncthreads();
@@ -223,6 +336,7 @@ __device__ void res_queue(const ResArgs& a) {
     if (n >= nphase * nb) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     const unsigned ph = n / nb, b = n - ph * nb;
+    SquareAcc acc;
     const unsigned grp_id = b * RES_NT + threadIdx.x;
     if (grp_id < ngroups) {
       const int row = (int)(grp_id / (unsigned)ng), g4 = (int)(grp_id - (unsigned)(row * ng));
@@ -263,24 +377,34 @@ __device__ void res_queue(const ResArgs& a) {
                                                    c3s * south[q] + c4l * pu + c4s * pd - rr[q]) -
                                             pc);
             own[base + q] = pc + reltmp;
+            if constexpr (RESID) acc.add(reltmp * reltmp, sLimb);
           }
         }
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if constexpr (RESID) {
+      acc.flush(sLimb);
+      const unsigned it = ph > 0u ? (ph - 1u) / (2u * per) + 1u : 0u;  // the iteration, from 1
+      if (ph > 0u && res_add_limbs(a, sLimb, &a.ctl->added, it * 2u * per * nb, sSum, &sFlag) &&
+          threadIdx.x == 0)
+        res_decide(a, sSum, it);
+    }
     __syncthreads();
     if (threadIdx.x == 0) atomicAdd(&a.ctl->tasks, 1u);
   }
 }
 
 // TK levels per thread; NS: LDS entries per level (threads used, at most RES_NT); KS1: one
-// level block per workgroup.
-template <int TK, int NS, bool KS1>
+// level block per workgroup; RESID: with the residual and the early exit.
+template <int TK, int NS, bool KS1, bool RESID>
 __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
   __shared__ float4 sP[2][TK][NS];
   __shared__ float4 sC[KS1 ? TK : RES_KWMAX];  // cn1, cn4l, cn4s of the workgroup's levels
   __shared__ __attribute__((aligned(16))) float sJ[2][res_jn(TK) * RES_NT];  // the rows across the south / north face, one colour
-  __shared__ unsigned sCtl[2];
+  __shared__ unsigned sCtl[3];
+  __shared__ u64 sLimb[RESID ? NLIMB : 1];
+  __shared__ int64_t sSum[RESID ? NLIMB : 1];
   const Dims d = a.d;
   const SplitSOR sp = a.sp;
   const int t = threadIdx.x;
@@ -317,11 +441,13 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
   }
   __syncthreads();
   if (sCtl[0] != RES_GO) {
-    res_queue(a);
+    res_queue<RESID>(a);
     res_leave(a);
     return;
   }
   const unsigned base_tag = sCtl[1];
+  if (RESID && t < NLIMB) sLimb[t] = 0;
+  SquareAcc acc;
 
   const int ng = sp.nr >> 2;
   const int blk = rj * ng;  // threads per level block
@@ -536,6 +662,7 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
         const float pcv[4] = {pc4.x, pc4.y, pc4.z, pc4.w}, rv[4] = {rr4.x, rr4.y, rr4.z, rr4.w};
         const float nv[4] = {xn.x, xn.y, xn.z, xn.w}, sv[4] = {xs.x, xs.y, xs.z, xs.w};
         const float uv[4] = {up.x, up.y, up.z, up.w}, dv[4] = {dn.x, dn.y, dn.z, dn.w};
+        const bool row1 = b ? s1 : !s1;  // the row's first cell is i = 1
         z[0] = w0[b] ? pcv[0] : z[0];
 #pragma unroll
         for (int q = 0; q < 4; ++q) z[q + 1] = eq[b][q] ? pcv[q] : z[q + 1];
@@ -547,6 +674,10 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
                             cc.z * dv[q] - rv[q]) -
                     pcv[q]);
           out[q] = pcv[q] + reltmp;
+          if constexpr (RESID) {  // (the padding past i = ip is no cell)
+            const int i = (row1 ? 1 : 2) + 2 * (4 * grp + q);
+            acc.add(i <= d.ip ? reltmp * reltmp : 0.0f, sLimb);
+          }
         }
         const float4 o4 = make_float4(out[0], out[1], out[2], out[3]);
         p[C][l] = o4;
@@ -607,9 +738,24 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
     }
     lds_only_barrier();
   };
-  for (int it = 0; it < a.nmaxp; ++it) {
+  for (unsigned it = 0; it < (unsigned)a.nmaxp; ++it) {
     half(std::integral_constant<int, 1>{}, 2u * it);
     half(std::integral_constant<int, 0>{}, 2u * it + 1u);
+    if constexpr (RESID) {  // the residual of the iteration, one decision for all workgroups
+      acc.flush(sLimb);
+      if (res_add_limbs(a, sLimb, &a.ctl->added, (unsigned)nwg * (it + 1u), sSum, &sCtl[2])) {
+        if (t == 0) sCtl[2] = res_decide(a, sSum, it + 1u);
+      } else if (t == 0) {
+        unsigned dec;
+        while ((dec = agent_load(&a.ctl->decided)) >> 1 < it + 1u && budget > 0) {
+          --budget;
+          __builtin_amdgcn_s_sleep(1);
+        }
+        sCtl[2] = dec;
+      }
+      __syncthreads();
+      if (sCtl[2] & 1u) break;
+    }
   }
 
   if (active) {
@@ -701,21 +847,28 @@ void res_free(ResBuf& b) {
 }
 
 namespace {
-template <int TK>
+template <int TK, bool RESID>
 void launch_tk(hipStream_t st, const ResArgs& a) {
   constexpr int NS = res_ns(TK);
+  const dim3 grid(a.pl.nwg()), blk(RES_NT);
   if (a.pl.ks == 1)
-    hipLaunchKernelGGL((k_sor_resident<TK, NS, true>), dim3(a.pl.nwg()), dim3(RES_NT), 0, st, a);
+    hipLaunchKernelGGL((k_sor_resident<TK, NS, true, RESID>), grid, blk, 0, st, a);
   if constexpr (TK <= RES_TK_KS)
-    if (a.pl.ks > 1)
-      hipLaunchKernelGGL((k_sor_resident<TK, NS, false>), dim3(a.pl.nwg()), dim3(RES_NT), 0, st, a);
+    if (a.pl.ks > 1) hipLaunchKernelGGL((k_sor_resident<TK, NS, false, RESID>), grid, blk, 0, st, a);
+}
+template <int TK>
+void launch_tk(hipStream_t st, const ResArgs& a) {
+  if (a.slots)
+    launch_tk<TK, true>(st, a);
+  else
+    launch_tk<TK, false>(st, a);
 }
 }  // namespace
 
 void launch_sor_resident(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Physics ph, int nmaxp,
-                         const DevScalars* sc, int sub_rhsav, int sub_pav, float* rout0,
-                         float* rout1, const ResPlan& pl, const ResBuf& b, long wait_ticks) {
-  ResArgs a{d, g, sp, ph.omega, nmaxp, sc, sub_rhsav, sub_pav, {rout0, rout1}, pl,
+                         DevScalars* sc, int sub_rhsav, int sub_pav, float* rout0, float* rout1,
+                         int64_t* resid_slots, const ResPlan& pl, const ResBuf& b, long wait_ticks) {
+  ResArgs a{d, g, sp, ph.omega, nmaxp, sc, sub_rhsav, sub_pav, {rout0, rout1}, ph.pjuge, resid_slots, pl,
             b.kslot, b.jslot, b.seam, b.ctl, wait_ticks};
   switch (pl.tk) {
     case 1: launch_tk<1>(st, a); break;

@@ -2,7 +2,7 @@
 bit: cuts with one and several workgroups along j and k, partial top level blocks and last rows,
 colour rows with padding, odd jp (the periodic seam joins cells of one colour), the largest
 number of levels per thread; the queue form that serves it when its workgroups cannot all be
-resident; and two handles taking turns on one device."""
+resident; two handles taking turns on one device; and the residual with the early exit."""
 import ctypes
 
 import numpy as np
@@ -15,9 +15,9 @@ pytestmark = pytest.mark.gpu
 FIELDS = ("p", "u", "v", "w", "rhs")
 
 
-def _handle(dims, nmaxp, sweeps, dx=4.0):
+def _handle(dims, nmaxp, sweeps, dx=4.0, pjuge=0.0):
     from les_halo_amd import LES, inputs
-    L = LES(*dims, **common.REF_PHYS, omega=1.5, pjuge=0.0, nmaxp=nmaxp)
+    L = LES(*dims, **common.REF_PHYS, omega=1.5, pjuge=pjuge, nmaxp=nmaxp)
     L.load_case(inputs.make_case(*dims, seed=5, hmax=20.0, dx=dx))
     L.ifdata()
     if sweeps:
@@ -81,3 +81,36 @@ def test_two_handles_take_turns():
         _same(h, hs[2])
     for h in hs:
         h.close()
+
+
+# pjuge: never met; just above the residual of iteration 4 of the first step
+@pytest.mark.parametrize("queue", [False, True])
+@pytest.mark.parametrize("dims", [(16, 12, 10), (48, 48, 32), (35, 27, 19), (150, 44, 61),
+                                  (147, 133, 61), (300, 300, 90)])
+def test_early_exit_equals_colour_sweeps(dims, queue):
+    from les_halo_amd._lib import lib
+    if queue and dims[0] > 100:
+        pytest.skip("the queue form is covered on the small grids")
+    probe = _handle(dims, 4, True, pjuge=1e-30)
+    probe.run(1, 1)
+    s4 = probe.scalars()["sor"]
+    probe.close()
+    for pjuge in (1e-30, float(np.float32(s4) * np.float32(1.0001))):
+        print(dims, queue, pjuge, flush=True)
+        a, b = _handle(dims, 9, False, pjuge=pjuge), _handle(dims, 9, True, pjuge=pjuge)
+        if queue:
+            assert lib().les_internal_sor_wait(a.h, ctypes.c_long(-1)) == 0
+        for n, m in ((1, 1), (2, 3)):  # eager, then graph replays
+            a.run(n, m)
+            b.run(n, m)
+            sa, sb = a.scalars(), b.scalars()
+            if n == 1:
+                assert sb["sor_iters"] == (9 if pjuge == 1e-30 else 4), sb
+            assert sa == sb
+            _same(a, b)
+        a.press_sor_solve()
+        b.press_sor_solve()
+        assert a.scalars() == b.scalars()
+        _same(a, b, ("p",))
+        a.close()
+        b.close()
