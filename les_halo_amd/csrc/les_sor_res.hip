@@ -45,8 +45,11 @@
 // 9 levels): 2.0 us computing (77 vector instructions a group of four cells, two wavefronts per
 // SIMD), 0.9 us more with k faces only, 5.0 us with both; memory is read once and written once
 // per solve.  50 iterations, measured with the scatter and gather of p around them: 300x300x90
-// 592 us against 50 x 20.5 us for k_sor_iter; 150x150x90 303 against 50 x 11.7; 32x24x16 133
-// against 50 x 8.3; 147x133x61 (odd jp) about 320 against 100 x (9.2 + 4.9) + 50 x 4.6 in place.
+// 592 us against 50 x 20.5 us for k_sor_iter; 150x150x90 282 against 50 x 11.7; 32x24x16 133
+// against 50 x 8.3; 147x133x61 (odd jp) about 250 against 100 x (9.2 + 4.9) + 50 x 4.6 in place.
+// With the residual (50 iterations): 1087, 694 and 299 us against 2109, 1471 and 1232 for the
+// residual-summing sweeps; what it adds is one all-workgroup hop an iteration (about 3 us, on the
+// smallest grid) and the sums' instructions.
 #include <algorithm>
 
 #include "les_sor_res.h"
@@ -56,8 +59,10 @@ namespace les {
 constexpr int RES_WGMAX = 1024;  // (no device has that many CUs)
 struct ResCtl {
   unsigned arrive, state, done, base, ticket, tasks;
-  // the residual: workgroups that have added theirs, iterations decided (times 2, plus 1: stop)
+  // the residual: workgroups that have added their exact sums, last iteration decided from them
+  // (times 2, plus 1: stop); each workgroup's sum of an iteration as two tagged words
   unsigned added, decided;
+  unsigned long long sums[2][2][RES_WGMAX];
   unsigned xcd[RES_WGMAX];  // the XCD each workgroup of the launch is on
 };
 
@@ -181,41 +186,90 @@ __device__ __forceinline__ void lds_only_barrier() {
   __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// Exact sum of the residual's terms reltmp**2 (never negative) of one thread and iteration: a term
-// m 2^(s-149) goes, shifted to its limb's origin, into one of three 64-bit sums for three limbs
-// next to each other (at most 2 * 4 * RES_TKMAX terms below 2^56 each: no overflow), the rare
-// others straight into the workgroup's limbs.  The integers added are those of ThreadAcc.
+// Exact sum of the residual's terms x = reltmp**2 of one thread and iteration.  Two FP64
+// accumulators start at 1.5 * 2^52 units and stay in that binade, so one unit is their last place:
+// 2^E0 and 2^E1, E0 = E1 + 45.  The first takes x rounded to its unit, the second what that left,
+// which is exact for x a multiple of 2^E1 below 2^(E1 + 89): |left| <= 2^(E1 + 44), and 8 * RES_TKMAX
+// terms move either accumulator by less than 2^51 units.  Every x from 2^(E1 + 23) on is such a
+// multiple; the others (few, E1 follows the sum of the iteration before) go to the workgroup's
+// limbs in LDS one by one, with their group's others.  Four FP64 additions a cell; with integer sums of the terms' 64-bit
+// parts an iteration at 300x300x90 took 32.1 us, now 20.0 (10.0 without the residual).
 struct SquareAcc {
-  u64 a0 = 0, a1 = 0, a2 = 0;
-  int base = -1;
-  __device__ __forceinline__ void add(float x, u64* lds) {
-    const unsigned b = __float_as_uint(x), e = b >> 23;  // sign 0
-    unsigned m = b & 0x7fffffu;
-    if (e) m |= 0x800000u;
-    if (e >= 0xffu) m = 0u;  // inf and nan are not summed
-    const int s = max((int)e, 1) - 1;
-    const u64 v = (u64)m << (s & 31);
-    if (base < 0 && m) base = min(max((s >> 5) - 1, 0), NLIMB - 4);
-    const int d = (s >> 5) - base;
-    a0 += d == 0 ? v : 0;
-    a1 += d == 1 ? v : 0;
-    a2 += d == 2 ? v : 0;
-    if ((d < 0 || d > 2) && m) {
-      atomicAdd(&lds[s >> 5], v & 0xffffffffull);
-      atomicAdd(&lds[(s >> 5) + 1], v >> 32);
+  double a0, a1;
+  int e1;           // uniform
+  unsigned lo, hi;  // bit patterns taken: lo <= bits < hi, and zero
+  static __device__ __forceinline__ double bias(int e) {  // 1.5 * 2^(52 + e)
+    return __longlong_as_double(((long long)(1023 + 52 + e) << 52) | 0x8000000000000ll);
+  }
+  // E1 for terms up to about 8 times 'sum'
+  __device__ __forceinline__ void start(double sum) {
+    const int e = (int)((__double_as_longlong(sum) >> 52) & 0x7ff) - 1023;
+    e1 = __builtin_amdgcn_readfirstlane(min(max(e + 4 - 89, -149), 39));
+    const int l = e1 + 23;
+    lo = e1 == -149 ? 1u : l >= -126 ? (unsigned)(l + 127) << 23 : 1u << (l + 149);
+    hi = min((unsigned)(e1 + 89 + 127) << 23, 0x7f800000u);
+    a0 = bias(e1 + 45);
+    a1 = bias(e1);
+  }
+  // four terms; one outside the range sends all four to the limbs
+  __device__ __forceinline__ void add4(const float (&x)[4], u64* limbs) {
+    unsigned most = 0u, least = ~0u;  // (zeros pass: least holds bits - 1)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      most = max(most, __float_as_uint(x[q]));
+      least = min(least, __float_as_uint(x[q]) - 1u);
+    }
+    if (most < hi && least >= lo - 1u) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const double v = (double)x[q], s = a0 + v;
+        a1 += v - (s - a0);
+        a0 = s;
+      }
+    } else {
+      TermParts t;
+#pragma unroll 1
+      for (int q = 0; q < 4; ++q)
+        if (split_term(q == 0 ? x[0] : q == 1 ? x[1] : q == 2 ? x[2] : x[3], t)) {
+          atomicAdd(&limbs[t.limb], (u64)t.lo);
+          atomicAdd(&limbs[t.limb + 1], (u64)t.hi);
+        }
     }
   }
-  // every lane of the wavefront together
-  __device__ __forceinline__ void flush(u64* lds) {
-    ThreadAcc t;
-    t.base = base;
-    t.r0 = (int64_t)(a0 & 0xffffffffull);
-    t.r1 = (int64_t)((a0 >> 32) + (a1 & 0xffffffffull));
-    t.r2 = (int64_t)((a1 >> 32) + (a2 & 0xffffffffull));
-    t.r3 = (int64_t)(a2 >> 32);
-    t.flush(lds);
-    a0 = a1 = a2 = 0;
-    base = -1;
+  // into the workgroup's units[2]; every lane of the wavefront together
+  __device__ __forceinline__ void flush(u64* units) const {
+    long long n0 = __double_as_longlong(a0) - __double_as_longlong(bias(e1 + 45));
+    long long n1 = __double_as_longlong(a1) - __double_as_longlong(bias(e1));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      n0 += __shfl_xor(n0, o);
+      n1 += __shfl_xor(n1, o);
+    }
+    if (__lane_id() == 0) {
+      atomicAdd(&units[0], (u64)n0);
+      atomicAdd(&units[1], (u64)n1);
+    }
+  }
+  // one thread: the workgroup's sum, rounded
+  __device__ __forceinline__ double value(const u64* units, const u64* limbs) const {
+    double v = ldexp((double)(long long)units[0], e1 + 45) + ldexp((double)(long long)units[1], e1);
+#pragma unroll
+    for (int q = 0; q < NLIMB; ++q) v += ldexp((double)(long long)limbs[q], 32 * q - 149);
+    return v;
+  }
+  // one thread: the workgroup's units into its limbs
+  __device__ __forceinline__ void fold(u64* units, u64* limbs) const {
+    for (int w = 0; w < 2; ++w) {
+      const long long n = (long long)units[w];
+      const int off = e1 + (w ? 0 : 45) + 149;
+      const long long part[2] = {n & 0xffffffffll, n >> 32};
+      for (int q = 0; q < 2; ++q) {
+        const int at = (off >> 5) + q;
+        const long long y = (long long)((u64)part[q] << (off & 31));
+        limbs[at] += (u64)(y & 0xffffffffll);
+        if (at + 1 < NLIMB) limbs[at + 1] += (u64)(y >> 32);  // (past the last limb: no bits)
+      }
+    }
   }
 };
 
@@ -336,7 +390,8 @@ __device__ void res_queue(const ResArgs& a) {
     if (n >= nphase * nb) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     const unsigned ph = n / nb, b = n - ph * nb;
-    SquareAcc acc;
+    ThreadAcc acc;
+    acc.init();
     const unsigned grp_id = b * RES_NT + threadIdx.x;
     if (grp_id < ngroups) {
       const int row = (int)(grp_id / (unsigned)ng), g4 = (int)(grp_id - (unsigned)(row * ng));
@@ -403,7 +458,9 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
   __shared__ float4 sC[KS1 ? TK : RES_KWMAX];  // cn1, cn4l, cn4s of the workgroup's levels
   __shared__ __attribute__((aligned(16))) float sJ[2][res_jn(TK) * RES_NT];  // the rows across the south / north face, one colour
   __shared__ unsigned sCtl[3];
-  __shared__ u64 sLimb[RESID ? NLIMB : 1];
+  // the residual's exact sum (by the iteration's parity) and the sum of all workgroups' by wavefront
+  __shared__ u64 sLimb[2][RESID ? NLIMB : 1], sUnit[2][2];
+  __shared__ double sWave[RES_NT / 64];
   __shared__ int64_t sSum[RESID ? NLIMB : 1];
   const Dims d = a.d;
   const SplitSOR sp = a.sp;
@@ -446,7 +503,10 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
     return;
   }
   const unsigned base_tag = sCtl[1];
-  if (RESID && t < NLIMB) sLimb[t] = 0;
+  if constexpr (RESID) {
+    if (t < 2 * NLIMB) sLimb[t / NLIMB][t % NLIMB] = 0;
+    if (t < 4) sUnit[t >> 1][t & 1] = 0;
+  }
   SquareAcc acc;
 
   const int ng = sp.nr >> 2;
@@ -666,7 +726,9 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
         z[0] = w0[b] ? pcv[0] : z[0];
 #pragma unroll
         for (int q = 0; q < 4; ++q) z[q + 1] = eq[b][q] ? pcv[q] : z[q + 1];
-        float out[4];
+        float out[4], sq[4];
+        // entries of the group that are cells (the padding past i = ip is none)
+        const int ncell = RESID ? ((d.ip - (row1 ? 1 : 2)) >> 1) + 1 - 4 * grp : 0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const float reltmp =
@@ -674,11 +736,9 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
                             cc.z * dv[q] - rv[q]) -
                     pcv[q]);
           out[q] = pcv[q] + reltmp;
-          if constexpr (RESID) {  // (the padding past i = ip is no cell)
-            const int i = (row1 ? 1 : 2) + 2 * (4 * grp + q);
-            acc.add(i <= d.ip ? reltmp * reltmp : 0.0f, sLimb);
-          }
+          if constexpr (RESID) sq[q] = q < ncell ? reltmp * reltmp : 0.0f;
         }
+        if constexpr (RESID) acc.add4(sq, sLimb[h >> 1 & 1u]);
         const float4 o4 = make_float4(out[0], out[1], out[2], out[3]);
         p[C][l] = o4;
         sP[C][l][t] = o4;
@@ -738,23 +798,63 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
     }
     lds_only_barrier();
   };
+  if constexpr (RESID) acc.start(1.0);
+  unsigned nexact = 0u;
   for (unsigned it = 0; it < (unsigned)a.nmaxp; ++it) {
     half(std::integral_constant<int, 1>{}, 2u * it);
     half(std::integral_constant<int, 0>{}, 2u * it + 1u);
-    if constexpr (RESID) {  // the residual of the iteration, one decision for all workgroups
-      acc.flush(sLimb);
-      if (res_add_limbs(a, sLimb, &a.ctl->added, (unsigned)nwg * (it + 1u), sSum, &sCtl[2])) {
-        if (t == 0) sCtl[2] = res_decide(a, sSum, it + 1u);
-      } else if (t == 0) {
-        unsigned dec;
-        while ((dec = agent_load(&a.ctl->decided)) >> 1 < it + 1u && budget > 0) {
-          --budget;
-          __builtin_amdgcn_s_sleep(1);
-        }
-        sCtl[2] = dec;
-      }
+    if constexpr (RESID) {
+      // All workgroups exchange their sums, rounded to FP64, in one hop and add them up alike.
+      // Well above pjuge that settles it; near or below it, and after the last iteration (whose
+      // residual is kept), the exact sum decides.
+      const unsigned par = it & 1u, tag = base_tag + 1u + it;
+      acc.flush(sUnit[par]);
       __syncthreads();
-      if (sCtl[2] & 1u) break;
+      if (t < NLIMB) sLimb[par ^ 1u][t] = 0;
+      if (t < 2) sUnit[par ^ 1u][t] = 0;
+      double sum = 0.0;
+      if (t == 0) {
+        sum = acc.value(sUnit[par], sLimb[par]);
+        const u64 v = (u64)__double_as_longlong(sum);
+        if (nwg > 1) {
+          agent_store(&a.ctl->sums[par][0][wg], ((u64)tag << 32) | (v & 0xffffffffull));
+          agent_store(&a.ctl->sums[par][1][wg], ((u64)tag << 32) | (v >> 32));
+          sum = 0.0;
+        }
+      }
+      for (int w = t; nwg > 1 && w < nwg; w += RES_NT) {
+        u64 lo, hi;
+        for (;;) {
+          lo = agent_load(&a.ctl->sums[par][0][w]);
+          hi = agent_load(&a.ctl->sums[par][1][w]);
+          if (((unsigned)(lo >> 32) == tag && (unsigned)(hi >> 32) == tag) || budget <= 0) break;
+          --budget;
+        }
+        sum += __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffull)));
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+      if ((t & 63) == 0) sWave[t >> 6] = sum;
+      __syncthreads();
+      sum = 0.0;
+#pragma unroll
+      for (int w = 0; w < RES_NT / 64; ++w) sum += sWave[w];
+      if (it + 1u == (unsigned)a.nmaxp || !(sum > (double)a.pjuge * (1.0 + 1e-6))) {
+        if (t == 0) acc.fold(sUnit[par], sLimb[par]);
+        if (res_add_limbs(a, sLimb[par], &a.ctl->added, (unsigned)nwg * ++nexact, sSum, &sCtl[2])) {
+          if (t == 0) sCtl[2] = res_decide(a, sSum, it + 1u);
+        } else if (t == 0) {
+          unsigned dec;
+          while ((dec = agent_load(&a.ctl->decided)) >> 1 < it + 1u && budget > 0) {
+            --budget;
+            __builtin_amdgcn_s_sleep(1);
+          }
+          sCtl[2] = dec;
+        }
+        __syncthreads();
+        if (sCtl[2] & 1u) break;
+      }
+      acc.start(sum);
     }
   }
 

@@ -112,5 +112,12 @@ def test_early_exit_equals_colour_sweeps(dims, queue):
         b.press_sor_solve()
         assert a.scalars() == b.scalars()
         _same(a, b, ("p",))
+        r = a.download("rhs")
+        for scale in (1e9, 1e-9):  # terms above and below what the FP64 accumulators hold
+            for h in (a, b):
+                h.upload("rhs", (r * np.float32(scale)).astype(np.float32))
+                h.press_sor_solve()
+            assert a.scalars() == b.scalars()
+            _same(a, b, ("p",))
         a.close()
         b.close()
