@@ -7,11 +7,14 @@ Workload: the plain LES step at 300x300x90 FP32 (dx = dy = 4 m, dz = 2 m stretch
 A step is one pass of the whole time step (velnw .. press) over the domain, replayed from a
 captured HIP graph with every input already resident in HBM.
 
-Prints one JSON line: value = M cell-steps/s of the whole job; roofline = the dominant kernel
-(the fused SOR iteration, or one colour sweep where the grid does not allow it) timed live with
-HIP events on the library's stream, against the HBM peak, priced at the algorithmic bytes of
-one SOR iteration at the stage boundaries of press.f95 (two colour sweeps, 16 B per cell; the
-fused kernel's own compulsory 12 B per cell are reported beside it); ensemble = the batched
+Prints one JSON line: value = M cell-steps/s of the whole job; roofline = the step's
+largest kernel with its operands in HBM (velfg + feedbf) timed live with HIP events on the
+library's stream, against the HBM peak at its algorithmic 85 B per cell, and beside it the time of
+the solve, which runs in one launch with p and rhs held on the chip (k_sor_resident: bound by
+the exchange between CUs and by instruction issue, memory is read and written once); with
+--sor-tile, the fused SOR iteration set by hand, priced at the algorithmic bytes of one SOR
+iteration at the stage boundaries of press.f95 (two colour sweeps, 16 B per cell; the fused
+kernel's own compulsory 12 B per cell are reported beside it); ensemble = the batched
 leg: the 64 uneven members of the ensemble configuration advanced together, against the same
 members run one after another; cpu_baseline = the reference Fortran time loop (built from the
 reference sources by oracle/ref/build_ref.sh with the benchmark's SOR settings, serial) on a
@@ -32,6 +35,7 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 # algorithmic FP32 bytes per interior cell-step: velnw 40 + velfg/feedbf/calc_sm 89 + visc/adam 88
 # + rhs 28 + 50 SOR iterations at 16 B (two 8 B colour sweeps) + pav/adj 12
 B_STEP = 1057
+VELFG_B_PER_CELL = 85          # velfg + feedbf (vel2 inlined)
 SOR_SWEEP_B_PER_CELL = 8       # one colour sweep: r p 4 + r rhs 2 + w p 2
 SOR_ITER_B_PER_CELL = 16       # one SOR iteration at press.f95's stage boundaries: two sweeps
 SOR_ITER_FUSED_B_PER_CELL = 12  # the fused iteration's compulsory bytes: r p 4 + r rhs 4 + w p 4
@@ -362,10 +366,23 @@ def main():
     ms_per_step = secs / args.steps * 1e3
     value = cells * args.steps / secs / 1e6
 
-    # dominant kernel (the fused SOR iteration when the grid allows it, else the colour
-    # sweep), timed live with HIP events on the library's stream
+    # the largest kernel in memory (the fused SOR iteration where it is set by hand), timed live
+    # with HIP events on the library's stream
     compulsory = None
-    if tuning["sor_tile_j"] > 0:
+    solve_us = None
+    if not args.sor_tile:
+        kern_ms = L.time_kernel("velfg", 100)
+        bytes_launch = VELFG_B_PER_CELL * cells
+        kname = "k_velfg_xy<true>"
+        for _ in range(3):
+            L.press_sor_solve()
+        L.sync()
+        t0 = time.perf_counter()
+        for _ in range(20):
+            L.press_sor_solve()
+        L.sync()
+        solve_us = (time.perf_counter() - t0) / 20 * 1e6
+    elif tuning["sor_tile_j"] > 0:
         kern_ms = L.time_kernel("sor_iter", 100)
         bytes_launch = SOR_ITER_B_PER_CELL * cells
         compulsory = SOR_ITER_FUSED_B_PER_CELL * cells
@@ -385,6 +402,10 @@ def main():
                 "tile": [tuning["sor_tile_j"], tuning["sor_tile_k"]],
                 "tuned_iter_us": (round(tuning["sor_iter_ms"] * 1e3, 3)
                                   if tuning["sor_iter_ms"] is not None else None)}
+    if solve_us is not None:
+        roofline["solve"] = {"kernel": "k_sor_resident", "us": round(solve_us, 1),
+                             "bound": "exchange between CUs + instruction issue (on the chip)",
+                             "timed_with": "the scatter and gather of p around it"}
     if compulsory:
         # the fused kernel's own compulsory traffic (both colours of p and rhs read once, both
         # colours of p written once), priced the same way

@@ -395,7 +395,9 @@ int les_time_kernel(les_handle* h, int which, int reps, float* avg_ms);
 /* Autotuner (no counterpart in the reference, whose OpenCL launch shapes are fixed): times one
  * SOR iteration without residual as two colour sweeps and as the fused launch with every
  * workgroup tile (rows of j x levels of k), 'reps' iterations each, on this handle's grid, and
- * keeps the fastest for later solves (untuned handles use the two sweeps); then times the
+ * keeps the fastest (untuned handles use the two sweeps) for the solves that cannot be held on
+ * the chip in one launch: where they can (uniform horizontal grid, mirror-image p halos, up to
+ * about 9 million cells), that form is taken, tuned or not; then times the
  * velnw, calc_sm and viscous-term kernels with each of their workgroup shapes (64x4, 128x2,
  * 32x8, 256x1) and keeps the fastest of each.  Changes no simulation state (the arrays the
  * stencil trials update are saved and restored).  *out (may be NULL) receives the choice. */
@@ -410,7 +412,7 @@ typedef struct les_tuning {
   float stencil_ms[3];
 } les_tuning;
 int les_autotune(les_handle* h, int reps, les_tuning* out);
-/* Sets the SOR iteration form by hand: tile_j = 0 for two colour sweeps, else the fused launch
+/* Sets the SOR iteration form by hand (instead of the solve held on the chip): tile_j = 0 for two colour sweeps, else the fused launch
  * with tile_j (4, 8 or 16) rows of j and tile_k levels of k per workgroup. */
 int les_set_sor_tile(les_handle* h, int tile_j, int tile_k);
 
