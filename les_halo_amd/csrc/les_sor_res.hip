@@ -375,14 +375,14 @@ __device__ void res_queue(const ResArgs& a) {
       sTask = n;
       if (n < nphase * nb) {
         const unsigned need = n / nb * nb;
-        bool stop = false;  // (decided before the iteration's last task ends)
-        for (;;) {
-          const bool go = agent_load(&a.ctl->tasks) >= need;
-          if (RESID) stop = agent_load(&a.ctl->decided) & 1u;
-          if (go || stop) break;
+        while (agent_load(&a.ctl->tasks) < need) {
+          if (RESID && (agent_load(&a.ctl->decided) & 1u)) break;
           __builtin_amdgcn_s_sleep(4);
         }
-        if (stop) sTask = 0xffffffffu;
+        // An iteration is decided before its last task ends, so with that count seen first every
+        // later task sees a stop: 'decided' must not be loaded before 'tasks'.
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (RESID && (agent_load(&a.ctl->decided) & 1u)) sTask = 0xffffffffu;
       }
     }
     __syncthreads();

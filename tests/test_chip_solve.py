@@ -121,3 +121,24 @@ def test_early_exit_equals_colour_sweeps(dims, queue):
             _same(a, b, ("p",))
         a.close()
         b.close()
+
+
+def test_queue_form_ends_with_the_exit():
+    """Many tasks a sweep, the exit in the middle of the solve, again and again on one handle: no
+    task of a sweep past the exit may run."""
+    from les_halo_amd._lib import lib
+    dims = (96, 96, 60)
+    probe = _handle(dims, 3, True, pjuge=1e-30)
+    probe.run(1, 1)
+    pjuge = float(np.float32(probe.scalars()["sor"]) * np.float32(1.0001))
+    probe.close()
+    a, b = _handle(dims, 40, False, pjuge=pjuge), _handle(dims, 40, True, pjuge=pjuge)
+    assert lib().les_internal_sor_wait(a.h, ctypes.c_long(-1)) == 0
+    for n in range(1, 9):
+        a.run(n, 1)
+        b.run(n, 1)
+        assert a.scalars() == b.scalars()
+        assert n > 1 or a.scalars()["sor_iters"] == 3
+        _same(a, b)
+    a.close()
+    b.close()
