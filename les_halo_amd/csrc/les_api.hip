@@ -1986,6 +1986,11 @@ extern "C" int les_internal_sor_wait(les_handle* h, long ticks) {
   return LES_OK;
 }
 
+// Not part of the ABI: the number of tasks of the queue form.
+extern "C" int64_t les_internal_sor_tasks(int ip, int jp, int kp, int nmaxp) {
+  return (int64_t)res_queue_tasks(Dims{ip, jp, kp}, ((ip + 1) / 2 + 3) / 4 * 4, nmaxp);
+}
+
 extern "C" int les_set_sor_tile(les_handle* h, int tile_j, int tile_k) {
   if (!h) return LES_E_INVALID;
   if (tile_j == 0) {

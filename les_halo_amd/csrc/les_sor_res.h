@@ -18,6 +18,16 @@ struct ResPlan {
   __host__ __device__ int nwg() const { return njt * nkt; }
 };
 
+// The queue form: tasks of RES_NT groups per phase; the phases are the shifts, then one per sweep (odd
+// jp: two, the seam's copy first).  64 bits: any nmaxp is taken, and 500 000 iterations at
+// 300x300x90 pass 2^32 tasks.
+__host__ __device__ inline unsigned res_queue_blocks(const Dims& d, int nr) {
+  return ((unsigned)(nr / 4 * d.jp * d.kp) + RES_NT - 1) / RES_NT;
+}
+__host__ __device__ inline unsigned long long res_queue_tasks(const Dims& d, int nr, int nmaxp) {
+  return res_queue_blocks(d, nr) * (1ull + 2ull * nmaxp * (d.jp % 2 ? 2 : 1));
+}
+
 constexpr long RES_WAIT_TICKS = 30000;  // 0.3 ms of the 100 MHz clock
 
 struct ResCtl;  // device control block (les_sor_res.hip)

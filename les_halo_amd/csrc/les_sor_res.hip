@@ -58,7 +58,8 @@ namespace les {
 
 constexpr int RES_WGMAX = 1024;  // (no device has that many CUs)
 struct ResCtl {
-  unsigned arrive, state, done, base, ticket, tasks;
+  unsigned arrive, state, done, base;
+  unsigned long long ticket, tasks;  // the queue form's (phases x tasks can pass 32 bits)
   // the residual: workgroups that have added their exact sums, last iteration decided from them
   // (times 2, plus 1: stop); each workgroup's sum of an iteration as two tagged words
   unsigned added, decided;
@@ -339,8 +340,8 @@ __device__ __forceinline__ void res_leave(const ResArgs& a) {
   if (atomicAdd(&a.ctl->done, 1u) != n - 1u) return;
   agent_store(&a.ctl->base, agent_load(&a.ctl->base) + 2u * (unsigned)a.nmaxp + 2u);
   agent_store(&a.ctl->arrive, 0u);
-  agent_store(&a.ctl->ticket, 0u);
-  agent_store(&a.ctl->tasks, 0u);
+  agent_store(&a.ctl->ticket, (u64)0);
+  agent_store(&a.ctl->tasks, (u64)0);
   agent_store(&a.ctl->added, 0u);
   agent_store(&a.ctl->decided, 0u);
   agent_store(&a.ctl->done, 0u);
@@ -354,7 +355,8 @@ __device__ __forceinline__ void res_leave(const ResArgs& a) {
 // of an iteration's limbs decides before its task ends; after a stop the tasks left are void.
 template <bool RESID>
 __device__ void res_queue(const ResArgs& a) {
-  __shared__ unsigned sTask, sFlag;
+  __shared__ u64 sTask;
+  __shared__ unsigned sFlag;
   __shared__ u64 sLimb[NLIMB];
   __shared__ int64_t sSum[NLIMB];
   if (RESID && threadIdx.x < NLIMB) sLimb[threadIdx.x] = 0;
@@ -363,18 +365,18 @@ __device__ void res_queue(const ResArgs& a) {
   const int ng = sp.nr / 4, pl = sp.nr * sp.nj;
   const bool odd = d.jp & 1;
   const unsigned ngroups = (unsigned)(ng * d.jp * d.kp);
-  const unsigned nb = (ngroups + RES_NT - 1) / RES_NT;
+  const unsigned nb = res_queue_blocks(d, sp.nr);
   const unsigned per = odd ? 2u : 1u;
-  const unsigned nphase = 1u + 2u * (unsigned)a.nmaxp * per;
+  const u64 ntask = res_queue_tasks(d, sp.nr, a.nmaxp);
   const float rsh = a.sub_rhsav ? a.sc->rhsav : 0.0f, psh = a.sub_pav ? a.sc->pav_carry : 0.0f;
   const float c2l = a.g.cn2l[0], c2s = a.g.cn2s[0], c3l = a.g.cn3l[0], c3s = a.g.cn3s[0];
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) {
-      const unsigned n = atomicAdd(&a.ctl->ticket, 1u);
+      const u64 n = atomicAdd(&a.ctl->ticket, (u64)1);
       sTask = n;
-      if (n < nphase * nb) {
-        const unsigned need = n / nb * nb;
+      if (n < ntask) {
+        const u64 need = n / nb * nb;
         while (agent_load(&a.ctl->tasks) < need) {
           if (RESID && (agent_load(&a.ctl->decided) & 1u)) break;
           __builtin_amdgcn_s_sleep(4);
@@ -382,14 +384,15 @@ __device__ void res_queue(const ResArgs& a) {
         // An iteration is decided before its last task ends, so with that count seen first every
         // later task sees a stop: 'decided' must not be loaded before 'tasks'.
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        if (RESID && (agent_load(&a.ctl->decided) & 1u)) sTask = 0xffffffffu;
+        if (RESID && (agent_load(&a.ctl->decided) & 1u)) sTask = ~(u64)0;
       }
     }
     __syncthreads();
-    const unsigned n = sTask;
-    if (n >= nphase * nb) return;
+    const u64 n = sTask;
+    if (n >= ntask) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    const unsigned ph = n / nb, b = n - ph * nb;
+    const u64 ph = n / nb;
+    const unsigned b = (unsigned)(n - ph * nb);
     ThreadAcc acc;
     acc.init();
     const unsigned grp_id = b * RES_NT + threadIdx.x;
@@ -403,8 +406,7 @@ __device__ void res_queue(const ResArgs& a) {
           if (a.sub_rhsav) st4(a.rout[c] + base, sub4(ld4(sp.r[c] + base), rsh));
         }
       } else {
-        const unsigned h = (ph - 1u) / per;
-        const int c = (h & 1u) ? 0 : 1;
+        const int c = ((ph - 1u) / per & 1u) ? 0 : 1;
         float* own = sp.p[c];
         if (odd && (ph - 1u) % per == 0u) {  // seam rows before the sweep: j = 1, then j = jp
           if (j == 1) st4(a.seam + sp.nr * (2 * kk) + 4 * g4, ld4(own + base));
@@ -440,13 +442,13 @@ __device__ void res_queue(const ResArgs& a) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     if constexpr (RESID) {
       acc.flush(sLimb);
-      const unsigned it = ph > 0u ? (ph - 1u) / (2u * per) + 1u : 0u;  // the iteration, from 1
+      const unsigned it = ph > 0u ? (unsigned)((ph - 1u) / (2u * per)) + 1u : 0u;  // the iteration, from 1
       if (ph > 0u && res_add_limbs(a, sLimb, &a.ctl->added, it * 2u * per * nb, sSum, &sFlag) &&
           threadIdx.x == 0)
         res_decide(a, sSum, it);
     }
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&a.ctl->tasks, 1u);
+    if (threadIdx.x == 0) atomicAdd(&a.ctl->tasks, (u64)1);
   }
 }
 
