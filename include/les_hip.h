@@ -138,7 +138,10 @@ int les_destroy(les_handle* h);
 const char* les_last_error(const les_handle* h);
 /* Interior sizes of the handle's grid. */
 int les_get_dims(const les_handle* h, int* ip, int* jp, int* kp);
-/* Waits for all work queued on the handle's stream. */
+/* Waits for all work queued on the handle's stream.  LES_E_HIP also when a pressure solve held on
+ * the chip gave up waiting for its own workgroups (seconds without an answer; p is not valid then);
+ * les_download, les_get_scalars and the other calls that wait for the device report it too, the
+ * first of them once, and later solves take the other forms. */
 int les_sync(les_handle* h);
 
 /* Replace the oclWrite* and oclRead* calls of one array (Wrappers/module_LES_combined_ocl.f95:359-418,

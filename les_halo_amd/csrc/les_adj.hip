@@ -731,6 +731,7 @@ size_t state_bytes(const les_adj* h) {
 int check(les_adj* h) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return afail(h, LES_E_HIP, std::string("launch: ") + hipGetErrorString(e));
+  if (h->ph && les::solve_failed(h->ph) != LES_OK) return afail(h, LES_E_HIP, les_last_error(h->ph));
   return LES_OK;
 }
 
@@ -897,7 +898,7 @@ static int xfer(les_adj* h, int field, double* host, bool up, bool adj) {
       for (long q = 0; q < n; ++q) host[q] = tmp[q];
     }
   }
-  return LES_OK;
+  return check(h);
 }
 
 extern "C" int les_adj_upload(les_adj* h, int field, const double* host) {

@@ -82,6 +82,8 @@ struct les_handle {
   bool capturing = false;     // the step is being captured into the handle's graph
   bool graph_chip = false;    // the captured step runs the chip-resident solve
   long res_wait = RES_WAIT_TICKS;
+  int res_polls = RES_POLLS;
+  bool res_off = false;       // a solve failed: the other forms from then on
   int ncu = 0;
   // workgroup shapes of the point-wise stencil kernels (les_autotune; 0 = 64 x 4)
   int shp_velnw = 0, shp_sm = 0, shp_visc = 0;
@@ -151,6 +153,17 @@ void res_release(les_handle* h) {
     T.recorded = false;
   }
   res_free(h->rbuf);
+}
+
+// The handle's stream has been waited for: an error if one of its chip-resident solves gave up (once;
+// later solves take the other forms)
+int solve_state(les_handle* h) {
+  volatile ResHost* w = h->rbuf.host;
+  if (!w || !w->failed) return LES_OK;
+  w->failed = 0;
+  h->res_off = true;
+  h->graph_valid = false;
+  return fail(h, LES_E_HIP, "SOR solve: the workgroups stopped answering each other; p is not valid");
 }
 
 // 'launch' enqueues work with a chip-resident solve of h on stream st, in its turn
@@ -654,7 +667,7 @@ extern "C" int les_get_dims(const les_handle* h, int* ip, int* jp, int* kp) {
 extern "C" int les_sync(les_handle* h) {
   if (!h) return LES_E_INVALID;
   HIPCHK(h, hipStreamSynchronize(h->st));
-  return LES_OK;
+  return solve_state(h);
 }
 
 extern "C" int les_upload(les_handle* h, int field, const float* host) {
@@ -766,7 +779,7 @@ extern "C" int les_download(les_handle* h, int field, float* host) {
   if (field == LES_RHS) sync_rhs(h);
   HIPCHK(h, hipStreamSynchronize(h->st));
   HIPCHK(h, hipMemcpy(host, h->fld[field], (size_t)h->cnt[field] * sizeof(float), hipMemcpyDeviceToHost));
-  return LES_OK;
+  return solve_state(h);
 }
 
 extern "C" int les_device_ptr(les_handle* h, int field, void** dptr, int64_t* count) {
@@ -992,13 +1005,14 @@ bool use_split(const les_handle* h) {
 // choose it.
 bool chip_solve(les_handle* h, bool resid) {
   return !(resid && seq_sums(h)) && h->sp.uniform && h->p_consistent && h->cn1_separable && h->split_ok &&
-         !h->sor_form_set && h->cfg.nmaxp > 0 && res_ready(h);
+         !h->sor_form_set && !h->res_off && h->cfg.nmaxp > 0 && res_ready(h);
 }
 
 int launch_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_pav, bool resid) {
   auto go = [&]() {
     launch_sor_resident(h->st, h->d, grid_of(h), h->sp, ph, h->cfg.nmaxp, h->sc, sub_rhsav, sub_pav,
-                        h->ra[0], h->ra[1], resid ? h->rb.slots : nullptr, h->rplan, h->rbuf, h->res_wait);
+                        h->ra[0], h->ra[1], resid ? h->rb.slots : nullptr, h->rplan, h->rbuf, h->res_wait,
+                        h->res_polls);
     return check_launch(h);
   };
   if (h->capturing) {
@@ -1181,7 +1195,8 @@ int enqueue_press_mixed(les_handle* h) {
   launch_mx_pav_gather(h->st, d, g, F, h->sp, h->mx, h->sc);
   HIPCHK(h, hipStreamSynchronize(h->st));  // 'passes' lives on this stack frame
   h->p_consistent = true;
-  return check_launch(h);
+  if ((r = check_launch(h))) return r;
+  return solve_state(h);
 }
 
 // The resident split solve applies: the chip-resident form, or fused iterations in pairs without
@@ -1286,6 +1301,7 @@ void set_drag(les_handle* h, const float* cd) {
   h->graph_valid = false;
 }
 void set_p_consistent(les_handle* h, bool consistent) { h->p_consistent = consistent; }
+int solve_failed(les_handle* h) { return h ? solve_state(h) : LES_OK; }
 int step_external(les_handle* h, hipStream_t st, int n) {
   if (!h) return LES_E_INVALID;
   const hipStream_t own = h->st;
@@ -1815,7 +1831,7 @@ extern "C" int les_get_scalars(les_handle* h, les_scalars* out) {
     HIPCHK(h, hipMemcpy(&it, h->mx.cg + 6, sizeof(double), hipMemcpyDeviceToHost));
     out->cg_iters = (int)it;
   }
-  return LES_OK;
+  return solve_state(h);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1982,6 +1998,15 @@ extern "C" int les_time_kernel(les_handle* h, int which, int reps, float* avg_ms
 extern "C" int les_internal_sor_wait(les_handle* h, long ticks) {
   if (!h) return LES_E_INVALID;
   h->res_wait = ticks;
+  h->graph_valid = false;
+  return LES_OK;
+}
+
+// Not part of the ABI: how many unanswered polls of a sweep's waits end them; 0: none is answered.
+// For the test of a solve that gives up.
+extern "C" int les_internal_sor_polls(les_handle* h, int polls) {
+  if (!h) return LES_E_INVALID;
+  h->res_polls = polls;
   h->graph_valid = false;
   return LES_OK;
 }

@@ -319,6 +319,8 @@ float* field_ptr(::les_handle* h, int field);
 void set_drag(::les_handle* h, const float* cd);
 void set_p_consistent(::les_handle* h, bool consistent);
 int step_external(::les_handle* h, hipStream_t st, int n);
+// The stream these were enqueued on has been waited for: LES_E_HIP (once) if a solve gave up.
+int solve_failed(::les_handle* h);
 // the stages of that step before the pressure solve (velnw to visc/adam), for the adjoint
 // form's recomputation: u, v, w after velnw and the inflow (before the outflow) are copied to
 // u_pre, v_pre, w_pre, and uout to uout_dst (device pointers)

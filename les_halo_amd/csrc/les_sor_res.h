@@ -29,8 +29,14 @@ __host__ __device__ inline unsigned long long res_queue_tasks(const Dims& d, int
 }
 
 constexpr long RES_WAIT_TICKS = 30000;  // 0.3 ms of the 100 MHz clock
+constexpr int RES_POLLS = 1 << 22;      // unanswered polls of a sweep's waits: some seconds
 
 struct ResCtl;  // device control block (les_sor_res.hip)
+
+// What a solve tells the host, in pinned host memory
+struct ResHost {
+  unsigned failed;  // a solve gave up waiting: its p is NaN
+};
 
 // Face slots and control block of one handle (res_alloc / res_free)
 struct ResBuf {
@@ -38,6 +44,7 @@ struct ResBuf {
   unsigned long long* jslot = nullptr;
   float* seam = nullptr;
   ResCtl* ctl = nullptr;
+  ResHost* host = nullptr;
 };
 
 ResPlan res_plan(Dims d, int nr, int ncu);
@@ -48,9 +55,11 @@ void res_free(ResBuf& b);
 // sub_pav: DevScalars::pav_carry is taken off every p value read.  resid_slots (RedBuf::slots, zero):
 // with the residual of every iteration (DevScalars::sor, sor_iters) and the early exit; null:
 // without.  wait_ticks (100 MHz): how long the workgroups wait for each other to be resident
-// before the solve falls back to the queue form; negative: the queue form at once.
+// before the solve falls back to the queue form; negative: the queue form at once.  polls
+// (RES_POLLS): the bound of its later waits.
 void launch_sor_resident(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Physics ph, int nmaxp,
                          DevScalars* sc, int sub_rhsav, int sub_pav, float* rout0, float* rout1,
-                         int64_t* resid_slots, const ResPlan& pl, const ResBuf& b, long wait_ticks);
+                         int64_t* resid_slots, const ResPlan& pl, const ResBuf& b, long wait_ticks,
+                         int polls);
 
 }  // namespace les

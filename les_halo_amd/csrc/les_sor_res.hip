@@ -59,6 +59,8 @@ namespace les {
 constexpr int RES_WGMAX = 1024;  // (no device has that many CUs)
 struct ResCtl {
   unsigned arrive, state, done, base;
+  unsigned failed;  // a wait was given up in this launch
+  ResHost* host;    // what the host is told
   unsigned long long ticket, tasks;  // the queue form's (phases x tasks can pass 32 bits)
   // the residual: workgroups that have added their exact sums, last iteration decided from them
   // (times 2, plus 1: stop); each workgroup's sum of an iteration as two tagged words
@@ -95,6 +97,7 @@ struct ResArgs {
   float* seam;
   ResCtl* ctl;
   long wait_ticks;
+  int polls;  // most unanswered polls of a sweep's waits
 };
 
 template <class T>
@@ -136,19 +139,32 @@ __device__ __forceinline__ void face_store(u64* p, int stride, float4 x, unsigne
     for (int q = 0; q < 4; ++q) word_store(p + q * stride, v[q], tag, false);
   }
 }
-// The face's values once all four carry 'tag'.  The wait ends because every workgroup is
-// resident and a sweep waits only for the one before it; 'budget' bounds it all the same (a
-// thread that used it up stores NaN).
+// A poll left unanswered, and the word read again.  Waits end because every workgroup is resident and a
+// sweep waits only for the one before it; 'budget', the polls that a sweep's waits may leave
+// unanswered, bounds them all the same (seconds).  A thread that uses it up takes NaN for the
+// missing word, which spreads with the sweeps, waits no more, and says so at the end of the solve:
+// the host gets an error (ResHost::failed).
+__device__ __forceinline__ u64 poll_again(const u64* p, unsigned tag, int& budget) {
+  if (--budget > 0) return agent_load(p);
+  budget = 0;
+  return ((u64)tag << 32) | 0x7fc00000u;
+}
+// The face's values once all four carry 'tag'.
 template <int STRIDE>
 __device__ __forceinline__ float4 face_wait(Face4 f, const u64* p, unsigned tag, int& budget) {
   for (;;) {
     bool ok = true;
 #pragma unroll
     for (int q = 0; q < 4; ++q) ok = ok && (unsigned)(f.v[q] >> 32) == tag;
-    if (ok || budget <= 0) break;
-    --budget;
+    if (ok) break;
     __builtin_amdgcn_s_sleep(1);
-    f = face_load<STRIDE>(p);
+    if (--budget > 0) {
+      f = face_load<STRIDE>(p);
+    } else {
+      budget = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) f.v[q] = ((u64)tag << 32) | 0x7fc00000u;
+    }
   }
   return make_float4(__uint_as_float((unsigned)f.v[0]), __uint_as_float((unsigned)f.v[1]),
                      __uint_as_float((unsigned)f.v[2]), __uint_as_float((unsigned)f.v[3]));
@@ -338,7 +354,14 @@ __device__ __forceinline__ void res_leave(const ResArgs& a) {
   if (threadIdx.x != 0) return;
   const unsigned n = (unsigned)a.pl.nwg();
   if (atomicAdd(&a.ctl->done, 1u) != n - 1u) return;
-  agent_store(&a.ctl->base, agent_load(&a.ctl->base) + 2u * (unsigned)a.nmaxp + 2u);
+  const unsigned failed = agent_load(&a.ctl->failed), base = agent_load(&a.ctl->base);
+  if (failed) {
+    for (int q = 0; a.slots && q < RED_SLOTS * NLIMB; ++q) agent_store(a.slots + q, (int64_t)0);
+    agent_store(&a.sc->sor, __builtin_nanf(""));
+    __hip_atomic_store(&a.ctl->host->failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    agent_store(&a.ctl->failed, 0u);
+  }
+  agent_store(&a.ctl->base, base + 2u * (unsigned)a.nmaxp + 2u);
   agent_store(&a.ctl->arrive, 0u);
   agent_store(&a.ctl->ticket, (u64)0);
   agent_store(&a.ctl->tasks, (u64)0);
@@ -660,7 +683,7 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
   // the seam's colour 1 as of "sweep -2" (colour 0, "sweep -1", goes out with the first sweep)
   if (odd_jp) j_publish(std::integral_constant<int, 1>{}, base_tag, bufof(0u));
 
-  int budget = 1 << 22;
+  int budget = a.polls;
   struct Lds {  // a level's operands from LDS
     float4 n, s;
     float x;
@@ -672,6 +695,7 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
   auto half = [&](auto Cc, unsigned h) {
     constexpr int C = decltype(Cc)::value, O = 1 - C;
     const unsigned tagK = base_tag + 1u + h;  // tag of sweep h - 1
+    if (budget > 0) budget = a.polls;
     if (faceJ) {  // publish the rows at the j faces, take those across them into LDS
       j_publish(std::integral_constant<int, O>{}, tagK, bufof(h + 1u));
       const bool seamS = odd_jp && jt == 0, seamN = odd_jp && jt == njt - 1;
@@ -691,10 +715,8 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
       for (int f = 0; f < 2; ++f)
 #pragma unroll
         for (int i = 0; i < JN; ++i) {
-          while ((unsigned)(jw[f][i] >> 32) != (f ? tagN : tagS) && t + i * RES_NT < njw && budget > 0) {
-            --budget;
-            jw[f][i] = agent_load(word_at(a.jslot, (f ? inN : inS) + i * RES_NT * 8u, t8));
-          }
+          while ((unsigned)(jw[f][i] >> 32) != (f ? tagN : tagS) && t + i * RES_NT < njw)
+            jw[f][i] = poll_again(word_at(a.jslot, (f ? inN : inS) + i * RES_NT * 8u, t8), f ? tagN : tagS, budget);
           sJ[f][t + i * RES_NT] = __uint_as_float((unsigned)jw[f][i]);
         }
       lds_only_barrier();
@@ -825,13 +847,10 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
         }
       }
       for (int w = t; nwg > 1 && w < nwg; w += RES_NT) {
-        u64 lo, hi;
-        for (;;) {
-          lo = agent_load(&a.ctl->sums[par][0][w]);
-          hi = agent_load(&a.ctl->sums[par][1][w]);
-          if (((unsigned)(lo >> 32) == tag && (unsigned)(hi >> 32) == tag) || budget <= 0) break;
-          --budget;
-        }
+        u64 lo = agent_load(&a.ctl->sums[par][0][w]), hi = agent_load(&a.ctl->sums[par][1][w]);
+        while ((unsigned)(lo >> 32) != tag) lo = poll_again(&a.ctl->sums[par][0][w], tag, budget);
+        while ((unsigned)(hi >> 32) != tag) hi = poll_again(&a.ctl->sums[par][1][w], tag, budget);
+        if (budget <= 0) hi = 0x7ff80000u;  // NaN: to the exact sum's path
         sum += __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffull)));
       }
 #pragma unroll
@@ -861,7 +880,6 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
   }
 
   if (active) {
-    const float bad = __builtin_nanf("");
 #pragma unroll
     for (int l = 0; l < TK; ++l) {
       if (l >= nlev) continue;
@@ -869,7 +887,6 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
       for (int c = 0; c < 2; ++c) {
         const int i0 = first_of(c, j, k0 + l) + 8 * grp;
         float4 x = p[c][l];
-        if (budget <= 0) x = make_float4(bad, bad, bad, bad);
         if (i0 > d.ip) x.x = 0.0f;
         if (i0 + 2 > d.ip) x.y = 0.0f;
         if (i0 + 4 > d.ip) x.z = 0.0f;
@@ -877,6 +894,10 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
         st4(sp.p[c] + off0 + l * lstride, x);
       }
     }
+  }
+  if (budget <= 0) {
+    agent_store(&a.ctl->failed, 1u);
+    __builtin_amdgcn_s_waitcnt(0);  // before this workgroup is counted as done
   }
   res_leave(a);
 }
@@ -930,10 +951,13 @@ hipError_t res_alloc(Dims d, int nr, const ResPlan& pl, hipStream_t st, ResBuf& 
   if (e == hipSuccess) e = hipMalloc(&b.jslot, nj * sizeof(u64));
   if (e == hipSuccess) e = hipMalloc(&b.seam, ns * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&b.ctl, sizeof(ResCtl));
+  if (e == hipSuccess) e = hipHostMalloc(&b.host, sizeof(ResHost), hipHostMallocDefault);
+  if (e == hipSuccess) *b.host = ResHost{};
   if (e == hipSuccess) e = hipMemsetAsync(b.kslot, 0, nk * sizeof(u64), st);
   if (e == hipSuccess) e = hipMemsetAsync(b.jslot, 0, nj * sizeof(u64), st);
   ResCtl c0{};
   c0.base = 1u;
+  c0.host = b.host;
   if (e == hipSuccess) e = hipMemcpyAsync(b.ctl, &c0, sizeof c0, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) res_free(b);
@@ -945,6 +969,7 @@ void res_free(ResBuf& b) {
   if (b.jslot) hipFree(b.jslot);
   if (b.seam) hipFree(b.seam);
   if (b.ctl) hipFree(b.ctl);
+  if (b.host) hipHostFree(b.host);
   b = ResBuf{};
 }
 
@@ -969,9 +994,10 @@ void launch_tk(hipStream_t st, const ResArgs& a) {
 
 void launch_sor_resident(hipStream_t st, Dims d, Grid1D g, SplitSOR sp, Physics ph, int nmaxp,
                          DevScalars* sc, int sub_rhsav, int sub_pav, float* rout0, float* rout1,
-                         int64_t* resid_slots, const ResPlan& pl, const ResBuf& b, long wait_ticks) {
+                         int64_t* resid_slots, const ResPlan& pl, const ResBuf& b, long wait_ticks,
+                         int polls) {
   ResArgs a{d, g, sp, ph.omega, nmaxp, sc, sub_rhsav, sub_pav, {rout0, rout1}, ph.pjuge, resid_slots, pl,
-            b.kslot, b.jslot, b.seam, b.ctl, wait_ticks};
+            b.kslot, b.jslot, b.seam, b.ctl, wait_ticks, polls};
   switch (pl.tk) {
     case 1: launch_tk<1>(st, a); break;
     case 2: launch_tk<2>(st, a); break;

@@ -142,3 +142,50 @@ def test_queue_form_ends_with_the_exit():
         _same(a, b)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("pjuge", [0.0, 1e-30])
+@pytest.mark.parametrize("dims", [(48, 48, 32), (147, 133, 61)])
+def test_solve_that_gives_up_is_an_error(dims, pjuge):
+    """Waits that end unanswered (bounded to no second look here): the missing words are NaN, the next
+    call that waits for the device fails, and the handle goes on with the other forms, the sums'
+    scratch memory as clean as before."""
+    from les_halo_amd._lib import lib
+    from les_halo_amd.les import LESError
+    print(dims, pjuge, flush=True)
+    a, b = _handle(dims, 5, False, pjuge=pjuge), _handle(dims, 5, True, pjuge=pjuge)
+    for h in (a, b):
+        h.run(1, 3)
+    p, rhs = a.download("p"), a.download("rhs")
+    assert lib().les_internal_sor_polls(a.h, 0) == 0
+    a.press_sor_solve()
+    with pytest.raises(LESError, match="SOR solve"):
+        a.sync()
+    assert np.isnan(a.download("p")).any()
+    assert lib().les_internal_sor_polls(a.h, 1 << 22) == 0
+    for h in (a, b):
+        h.upload("p", p)
+        h.press_boundp()
+        h.upload("rhs", rhs)
+        h.press_sor_solve()
+        h.run(4, 2)
+    assert a.scalars() == b.scalars()
+    _same(a, b)
+    a.close()
+    b.close()
+
+
+def test_polls_are_counted_per_sweep():
+    """The bound of the waits is one sweep's: a solve of thousands of sweeps, whose unanswered polls
+    together pass it many times over, ends like the sweeps' one."""
+    from les_halo_amd._lib import lib
+    dims = (48, 48, 32)
+    a, b = _handle(dims, 3000, False), _handle(dims, 3000, True)
+    # one sweep takes 2 us and a poll some tenths: a few thousand polls are far from any sweep's
+    assert lib().les_internal_sor_polls(a.h, 1 << 13) == 0
+    for h in (a, b):
+        h.step(1)
+    a.sync()
+    _same(a, b)
+    a.close()
+    b.close()
