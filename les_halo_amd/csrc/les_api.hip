@@ -84,6 +84,11 @@ struct les_handle {
   long res_wait = RES_WAIT_TICKS;
   int res_polls = RES_POLLS;
   bool res_off = false;       // a solve failed: the other forms from then on
+  // for its turns with other handles (ResTurn, under its lock): the stream of the last launch with
+  // such a solve, and an event recorded after that launch if res_rec
+  hipStream_t res_st = nullptr;
+  hipEvent_t res_ev = nullptr;
+  bool res_rec = false;
   int ncu = 0;
   // workgroup shapes of the point-wise stencil kernels (les_autotune; 0 = 64 x 4)
   int shp_velnw = 0, shp_sm = 0, shp_visc = 0;
@@ -110,13 +115,14 @@ int fail(les_handle* h, int code, const std::string& msg) {
 // them has used that solve and their workgroups together exceed the CUs, whoever launches next
 // makes its stream wait for the last launch of another one.  (Kernels of other programs are
 // not seen here; the solve itself falls back to its queue form when they keep it from fitting.)
+// A handle by itself records no events (4 us a step); when a second one comes, it records what the
+// first has launched so far, on the first one's stream: none of these streams is captured without
+// the lock, and a handle leaves the list before its streams are destroyed.
 struct ResTurn {
   std::mutex m;
-  int handles = 0, wgs = 0;
+  std::vector<les_handle*> users;  // handles with chip-resident solves
+  int wgs = 0;
   les_handle* last = nullptr;
-  hipStream_t last_st = nullptr;
-  hipEvent_t ev = nullptr;
-  bool recorded = false;
 };
 constexpr int RES_DEVICES = 64;
 ResTurn g_turn[RES_DEVICES];
@@ -129,30 +135,28 @@ bool res_ready(les_handle* h) {
   if (h->capturing) return false;
   ResTurn& T = g_turn[h->cfg.device];
   std::lock_guard<std::mutex> lock(T.m);
-  if (!T.ev && hipEventCreateWithFlags(&T.ev, hipEventDisableTiming) != hipSuccess) T.ev = nullptr;
-  if (!T.ev || res_alloc(h->d, h->sp.nr, h->rplan, h->st, h->rbuf) != hipSuccess) {
+  if (!h->res_ev && hipEventCreateWithFlags(&h->res_ev, hipEventDisableTiming) != hipSuccess) h->res_ev = nullptr;
+  if (!h->res_ev || res_alloc(h->d, h->sp.nr, h->rplan, h->st, h->rbuf) != hipSuccess) {
     (void)hipGetLastError();
     h->rplan.tk = 0;
     return false;
   }
-  // the handles before this one may have launched without recording
-  if (T.last && !T.recorded) T.recorded = hipEventRecord(T.ev, T.last_st) == hipSuccess;
-  ++T.handles;
+  T.users.push_back(h);
   T.wgs += h->rplan.nwg();
   return true;
 }
 
 void res_release(les_handle* h) {
-  if (!h->rbuf.ctl) return;
-  ResTurn& T = g_turn[h->cfg.device];
-  std::lock_guard<std::mutex> lock(T.m);
-  --T.handles;
-  T.wgs -= h->rplan.nwg();
-  if (T.last == h) {  // its stream has been waited for
-    T.last = nullptr;
-    T.recorded = false;
+  if (h->rbuf.ctl) {  // its streams have been waited for
+    ResTurn& T = g_turn[h->cfg.device];
+    std::lock_guard<std::mutex> lock(T.m);
+    T.users.erase(std::find(T.users.begin(), T.users.end(), h));
+    T.wgs -= h->rplan.nwg();
+    if (T.last == h) T.last = nullptr;
+    res_free(h->rbuf);
   }
-  res_free(h->rbuf);
+  if (h->res_ev) hipEventDestroy(h->res_ev);
+  h->res_ev = nullptr;
 }
 
 // The handle's stream has been waited for: an error if one of its chip-resident solves gave up (once;
@@ -168,16 +172,28 @@ int solve_state(les_handle* h) {
 
 // 'launch' enqueues work with a chip-resident solve of h on stream st, in its turn
 template <class Launch>
-auto res_in_turn(les_handle* h, hipStream_t st, Launch&& launch) {
+hipError_t res_in_turn(les_handle* h, hipStream_t st, Launch&& launch) {
   ResTurn& T = g_turn[h->cfg.device];
   std::lock_guard<std::mutex> lock(T.m);
-  const bool share = T.handles > 1 && T.wgs > h->ncu;
-  if (share && T.last && T.last != h && T.recorded) (void)hipStreamWaitEvent(st, T.ev, 0);
-  auto r = launch();
+  const bool share = T.users.size() > 1 && T.wgs > h->ncu;
+  if (share)
+    for (les_handle* u : T.users) {
+      if (u == h || !u->res_st) continue;
+      const bool unseen = !u->res_rec;
+      hipError_t e = unseen ? hipEventRecord(u->res_ev, u->res_st) : hipSuccess;
+      if (e == hipSuccess) u->res_rec = true;
+      if (e == hipSuccess && (unseen || u == T.last)) e = hipStreamWaitEvent(st, u->res_ev, 0);
+      if (e != hipSuccess) return e;
+    }
+  hipError_t e = launch();
   T.last = h;
-  T.last_st = st;
-  T.recorded = share && hipEventRecord(T.ev, st) == hipSuccess;
-  return r;
+  h->res_st = st;
+  h->res_rec = false;
+  if (share && e == hipSuccess) {
+    e = hipEventRecord(h->res_ev, st);
+    h->res_rec = e == hipSuccess;
+  }
+  return e;
 }
 
 // Bounds table: lo/hi offsets relative to (0, ip, jp, kp) per dimension.
@@ -1013,13 +1029,15 @@ int launch_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_p
     launch_sor_resident(h->st, h->d, grid_of(h), h->sp, ph, h->cfg.nmaxp, h->sc, sub_rhsav, sub_pav,
                         h->ra[0], h->ra[1], resid ? h->rb.slots : nullptr, h->rplan, h->rbuf, h->res_wait,
                         h->res_polls);
-    return check_launch(h);
+    return hipGetLastError();
   };
   if (h->capturing) {
     h->graph_chip = true;
-    return go();
+    HIPCHK(h, go());
+  } else {
+    HIPCHK(h, res_in_turn(h, h->st, go));
   }
-  return res_in_turn(h, h->st, go);
+  return LES_OK;
 }
 
 // press.f95:87-115 on the Fortran arrays: colour sweep, boundp1 per colour, boundp2 per
@@ -1417,12 +1435,19 @@ int ensure_graph(les_handle* h) {
   h->graph = nullptr;
   (void)res_ready(h);  // no allocation inside the capture
   h->graph_chip = false;
-  HIPCHK(h, hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal));
-  h->capturing = true;
-  int r = enqueue_step(h, 2);
-  h->capturing = false;
+  int r;
   hipGraph_t gr = nullptr;
-  hipError_t e = hipStreamEndCapture(h->st, &gr);
+  hipError_t e;
+  {
+    // another thread's turn records on this stream: not while it is captured
+    std::unique_lock<std::mutex> lock;
+    if (h->rbuf.ctl) lock = std::unique_lock<std::mutex>(g_turn[h->cfg.device].m);
+    HIPCHK(h, hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal));
+    h->capturing = true;
+    r = enqueue_step(h, 2);
+    h->capturing = false;
+    e = hipStreamEndCapture(h->st, &gr);
+  }
   if (r) {
     if (gr) hipGraphDestroy(gr);
     return r;

@@ -189,3 +189,46 @@ def test_polls_are_counted_per_sweep():
     _same(a, b)
     a.close()
     b.close()
+
+
+def test_first_solves_while_another_thread_captures():
+    """Handles whose first solves on the chip fall into another thread's captures of its step:
+    neither may get into the other's capture, nor miss its turn."""
+    import threading
+
+    from les_halo_amd._lib import lib
+    dims, small = (96, 96, 20), (64, 64, 24)
+    a, b = _handle(dims, 4, False), _handle(dims, 4, True)
+    cs, c0 = [_handle(small, 4, False) for _ in range(12)], _handle(small, 4, True)
+    a.run(1, 3)
+    b.run(1, 3)
+    errs, done = [], threading.Event()
+
+    def first_solves():
+        try:
+            for c in cs:
+                c.run(1, 8)
+                c.sync()
+        except Exception as e:  # noqa: BLE001
+            errs.append(e)
+        finally:
+            done.set()
+
+    t = threading.Thread(target=first_solves)
+    t.start()
+    n = 4
+    try:
+        while not done.is_set() and n < 4000:
+            assert lib().les_internal_sor_polls(a.h, 1 << 22) == 0  # its graph is captured anew
+            a.run(n, 1)
+            n += 1
+    finally:
+        t.join()
+    assert not errs, errs
+    b.run(4, n - 4)
+    c0.run(1, 8)
+    _same(a, b)
+    for c in cs:
+        _same(c, c0)
+    for h in [a, b, c0] + cs:
+        h.close()
