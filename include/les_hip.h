@@ -418,6 +418,22 @@ int les_autotune(les_handle* h, int reps, les_tuning* out);
 /* Sets the SOR iteration form by hand (instead of the solve held on the chip): tile_j = 0 for two colour sweeps, else the fused launch
  * with tile_j (4, 8 or 16) rows of j and tile_k levels of k per workgroup. */
 int les_set_sor_tile(les_handle* h, int tile_j, int tile_k);
+/* How this handle's pressure solves run; waits for the handle's stream.  The solve held on the chip
+ * needs all its workgroups resident together.  Where they are not within 0.3 ms (another program's
+ * kernels, masked CUs) a solve runs through a queue of tasks in device memory, several times
+ * slower; after 16 of these in a row the handle takes the other forms (given_up). */
+typedef struct les_solve_info {
+  int on_chip;      /* the next solve is held on the chip */
+  int workgroups;   /* its cut of the grid (0: the grid does not fit): workgroups, their rows of j, */
+  int rows;         /* blocks of levels, and levels per block */
+  int level_blocks;
+  int levels;
+  int given_up;     /* it fits but is no longer used: see above, or a solve failed (les_sync) */
+  int64_t solves;   /* solves enqueued in that form */
+  int64_t queued;   /* ... that ran through the queue */
+  int64_t face_bytes; /* device memory held for it */
+} les_solve_info;
+int les_get_solve_info(les_handle* h, les_solve_info* out);
 
 /* ---- the reference's GPU host API (module_LES_combined_ocl) as single-handle drop-ins ---- */
 /* initialise_LES_kernel (Wrappers/module_LES_combined_ocl.f95:15-441), external wind profile

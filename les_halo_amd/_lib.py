@@ -38,6 +38,12 @@ class LesTuning(ctypes.Structure):
                 ("stencil_bx", c_int * 3), ("stencil_by", c_int * 3), ("stencil_ms", c_float * 3)]
 
 
+class LesSolveInfo(ctypes.Structure):
+    _fields_ = [("on_chip", c_int), ("workgroups", c_int), ("rows", c_int), ("level_blocks", c_int),
+                ("levels", c_int), ("given_up", c_int), ("solves", c_int64), ("queued", c_int64),
+                ("face_bytes", c_int64)]
+
+
 # every symbol declared in include/les_hip.h: name -> (restype, argtypes)
 H = c_void_p
 PROTOS = {
@@ -126,6 +132,7 @@ PROTOS = {
     "les_time_kernel": (c_int, [H, c_int, c_int, P_float]),
     "les_autotune": (c_int, [H, c_int, ctypes.POINTER(LesTuning)]),
     "les_set_sor_tile": (c_int, [H, c_int, c_int]),
+    "les_get_solve_info": (c_int, [H, ctypes.POINTER(LesSolveInfo)]),
     "les_ensemble_create": (c_int, [ctypes.POINTER(c_void_p), c_int, ctypes.POINTER(c_void_p)]),
     "les_ensemble_set_mode": (c_int, [c_void_p, c_int]),
     "les_ensemble_batched": (c_int, [c_void_p]),

@@ -83,7 +83,9 @@ struct les_handle {
   bool graph_chip = false;    // the captured step runs the chip-resident solve
   long res_wait = RES_WAIT_TICKS;
   int res_polls = RES_POLLS;
-  bool res_off = false;       // a solve failed: the other forms from then on
+  bool res_off = false;       // given up (RES_GIVE_UP, or a solve failed): the other forms are taken
+  unsigned res_row0 = 0;      // ... of the row seen, what came before les_autotune
+  int64_t res_solves = 0;     // such solves enqueued
   // for its turns with other handles (ResTurn, under its lock): the stream of the last launch with
   // such a solve, and an event recorded after that launch if res_rec
   hipStream_t res_st = nullptr;
@@ -170,6 +172,18 @@ int solve_state(les_handle* h) {
   return fail(h, LES_E_HIP, "SOR solve: the workgroups stopped answering each other; p is not valid");
 }
 
+// Solve after solve in the queue form: its workgroups do not get the device (another program, masked
+// CUs), and the other forms are faster.  Looked at before a step's or a solve's form is chosen.
+void res_check(les_handle* h) {
+  const volatile ResHost* w = h->rbuf.host;
+  if (!w || h->res_off || h->capturing) return;
+  const unsigned row = w->row;
+  h->res_row0 = std::min(h->res_row0, row);
+  if (row - h->res_row0 < RES_GIVE_UP) return;
+  h->res_off = true;
+  h->graph_valid = false;
+}
+
 // 'launch' enqueues work with a chip-resident solve of h on stream st, in its turn
 template <class Launch>
 hipError_t res_in_turn(les_handle* h, hipStream_t st, Launch&& launch) {
@@ -189,6 +203,7 @@ hipError_t res_in_turn(les_handle* h, hipStream_t st, Launch&& launch) {
   T.last = h;
   h->res_st = st;
   h->res_rec = false;
+  if (e == hipSuccess) ++h->res_solves;
   if (share && e == hipSuccess) {
     e = hipEventRecord(h->res_ev, st);
     h->res_rec = e == hipSuccess;
@@ -1019,10 +1034,11 @@ bool use_split(const les_handle* h) {
 // the reference's order of terms, and the form not set by hand.  Any parity of jp.  It is the
 // faster form wherever it fits (300x300x90: see the kernel's comment), so nothing is timed to
 // choose it.
-bool chip_solve(les_handle* h, bool resid) {
+bool chip_applies(const les_handle* h, bool resid) {
   return !(resid && seq_sums(h)) && h->sp.uniform && h->p_consistent && h->cn1_separable && h->split_ok &&
-         !h->sor_form_set && !h->res_off && h->cfg.nmaxp > 0 && res_ready(h);
+         !h->sor_form_set && !h->res_off && h->cfg.nmaxp > 0 && h->rplan.tk > 0;
 }
+bool chip_solve(les_handle* h, bool resid) { return chip_applies(h, resid) && res_ready(h); }
 
 int launch_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_pav, bool resid) {
   auto go = [&]() {
@@ -1089,6 +1105,7 @@ int enqueue_sor_split_loop(les_handle* h, bool allow_exit = true, const Physics*
 
 int enqueue_sor_solve(les_handle* h) {
   STAGE_BEGIN(h);
+  res_check(h);
   int r;
   if (use_split(h) || chip_solve(h, h->ph.pjuge > 0.0f)) {
     launch_split_scatter(h->st, d, F, h->sp, h->sc, 0);
@@ -1111,6 +1128,7 @@ namespace les {
 // init.f95 form) and, up to the caller, mirror-consistent halos of p on entry.
 int sor_solve_external(les_handle* h, hipStream_t st, float* p, float* rhs) {
   if (!h || !p || !rhs) return LES_E_INVALID;
+  res_check(h);
   h->sp_p_current = false;  // the split copy takes this solve's arrays
   if (!(h->d.jp % 2 == 0 && h->cn1_separable && h->split_ok))
     return fail(h, LES_E_STATE, "split solve does not apply to this grid");
@@ -1269,6 +1287,7 @@ int enqueue_press_resident(les_handle* h) {
 // press.f95:49-146
 int enqueue_press(les_handle* h) {
   STAGE_BEGIN(h);
+  res_check(h);
   if (h->cfg.precision == LES_PREC_MIXED) return enqueue_press_mixed(h);
   if (resident_applies(h)) return enqueue_press_resident(h);
   h->sp_p_current = false;
@@ -1479,6 +1498,7 @@ void after_replays(les_handle* h) {
 extern "C" int les_run(les_handle* h, int n0, int nsteps) {
   if (!h || nsteps < 0) return LES_E_INVALID;
   int r;
+  res_check(h);
   run_eager_prefix(h, n0, nsteps, r);
   if (r) return r;
   if (nsteps == 0) return LES_OK;
@@ -1796,6 +1816,7 @@ extern "C" int les_ensemble_run(les_ensemble* e, int n0, int nsteps) {
   for (int q = 0; q < nm; ++q) {
     les_handle* h = e->m[q];
     int r;
+    res_check(h);
     run_eager_prefix(h, n0, left[q], r);
     if (r) return r;
     if (left[q] > 0 && h->cfg.precision == LES_PREC_MIXED) return LES_E_STATE;
@@ -2016,6 +2037,26 @@ extern "C" int les_time_kernel(les_handle* h, int which, int reps, float* avg_ms
   hipEventDestroy(e1);
   *avg_ms = ms / (float)reps;
   return check_launch(h);
+}
+
+extern "C" int les_get_solve_info(les_handle* h, les_solve_info* out) {
+  if (!h || !out) return LES_E_INVALID;
+  HIPCHK(h, hipStreamSynchronize(h->st));
+  *out = les_solve_info{};
+  const volatile ResHost* w = h->rbuf.host;
+  res_check(h);
+  out->on_chip = chip_applies(h, h->ph.pjuge > 0.0f) ? 1 : 0;
+  if (h->rplan.tk > 0) {
+    out->workgroups = h->rplan.nwg();
+    out->rows = h->rplan.rj;
+    out->level_blocks = h->rplan.ks;
+    out->levels = h->rplan.tk;
+  }
+  out->given_up = h->res_off ? 1 : 0;
+  out->solves = h->res_solves;
+  out->queued = w ? (int64_t)w->queued : 0;
+  out->face_bytes = h->rbuf.ctl ? (int64_t)res_bytes(h->d, h->sp.nr, h->rplan) : 0;
+  return LES_OK;
 }
 
 // Not part of the ABI: how long (100 MHz ticks) the chip-resident solve's workgroups wait for each

@@ -29,13 +29,18 @@ __host__ __device__ inline unsigned long long res_queue_tasks(const Dims& d, int
 }
 
 constexpr long RES_WAIT_TICKS = 30000;  // 0.3 ms of the 100 MHz clock
+// So many solves in a row in the queue form, and the handle leaves this kernel: a few milliseconds
+// each at most, while one or two in a row are another kernel's that just ran.
+constexpr unsigned RES_GIVE_UP = 16;
 constexpr int RES_POLLS = 1 << 22;      // unanswered polls of a sweep's waits: some seconds
 
 struct ResCtl;  // device control block (les_sor_res.hip)
 
 // What a solve tells the host, in pinned host memory
 struct ResHost {
-  unsigned failed;  // a solve gave up waiting: its p is NaN
+  unsigned failed;  // a solve gave up waiting: words of its p are NaN
+  unsigned queued;  // solves that took the queue form, their workgroups not all resident in time
+  unsigned row;     // ... how many of the last ones in a row
 };
 
 // Face slots and control block of one handle (res_alloc / res_free)
@@ -50,6 +55,7 @@ struct ResBuf {
 ResPlan res_plan(Dims d, int nr, int ncu);
 hipError_t res_alloc(Dims d, int nr, const ResPlan& pl, hipStream_t st, ResBuf& b);
 void res_free(ResBuf& b);
+size_t res_bytes(Dims d, int nr, const ResPlan& pl);  // device memory of res_alloc
 // nmaxp SOR iterations (press.f95:87-115) on the split copy sp.p / sp.r in place.  sub_rhsav: sp.r
 // holds the raw rhs; rhsav is taken off every value read and the result written to rout.
 // sub_pav: DevScalars::pav_carry is taken off every p value read.  resid_slots (RedBuf::slots, zero):

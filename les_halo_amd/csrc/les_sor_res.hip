@@ -60,6 +60,7 @@ constexpr int RES_WGMAX = 1024;  // (no device has that many CUs)
 struct ResCtl {
   unsigned arrive, state, done, base;
   unsigned failed;  // a wait was given up in this launch
+  unsigned queued, row;  // launches that took the queue form; of these the last in a row
   ResHost* host;    // what the host is told
   unsigned long long ticket, tasks;  // the queue form's (phases x tasks can pass 32 bits)
   // the residual: workgroups that have added their exact sums, last iteration decided from them
@@ -349,12 +350,20 @@ __device__ inline bool res_add_limbs(const ResArgs& a, u64* lds, unsigned* count
 
 // The last workgroup to leave re-arms the control block for the next launch (stream order makes
 // it visible there).
-__device__ __forceinline__ void res_leave(const ResArgs& a) {
+__device__ __forceinline__ void res_leave(const ResArgs& a, bool queued) {
   __syncthreads();
   if (threadIdx.x != 0) return;
   const unsigned n = (unsigned)a.pl.nwg();
   if (atomicAdd(&a.ctl->done, 1u) != n - 1u) return;
   const unsigned failed = agent_load(&a.ctl->failed), base = agent_load(&a.ctl->base);
+  const unsigned row = agent_load(&a.ctl->row);
+  if (queued || row) {  // (the host's memory is written only where something changes)
+    const unsigned total = agent_load(&a.ctl->queued) + (queued ? 1u : 0u), r = queued ? row + 1u : 0u;
+    agent_store(&a.ctl->queued, total);
+    agent_store(&a.ctl->row, r);
+    __hip_atomic_store(&a.ctl->host->queued, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&a.ctl->host->row, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
   if (failed) {
     for (int q = 0; a.slots && q < RED_SLOTS * NLIMB; ++q) agent_store(a.slots + q, (int64_t)0);
     agent_store(&a.sc->sor, __builtin_nanf(""));
@@ -524,7 +533,7 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
   __syncthreads();
   if (sCtl[0] != RES_GO) {
     res_queue<RESID>(a);
-    res_leave(a);
+    res_leave(a, true);
     return;
   }
   const unsigned base_tag = sCtl[1];
@@ -899,7 +908,7 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
     agent_store(&a.ctl->failed, 1u);
     __builtin_amdgcn_s_waitcnt(0);  // before this workgroup is counted as done
   }
-  res_leave(a);
+  res_leave(a, false);
 }
 
 }  // namespace
@@ -943,10 +952,20 @@ ResPlan res_plan(Dims d, int nr, int ncu) {
   return best;
 }
 
+namespace {
+size_t kwords(const ResPlan& pl) { return (size_t)pl.nwg() * 2 * 2 * 4 * RES_NT; }
+size_t jwords(Dims d, const ResPlan& pl) {
+  return (size_t)pl.nwg() * (d.jp % 2 ? 2 : 1) * 2 * 2 * res_jn(pl.tk) * RES_NT;
+}
+size_t seam_floats(Dims d, int nr) { return (size_t)2 * d.kp * nr; }
+}  // namespace
+
+size_t res_bytes(Dims d, int nr, const ResPlan& pl) {
+  return (kwords(pl) + jwords(d, pl)) * sizeof(u64) + seam_floats(d, nr) * sizeof(float) + sizeof(ResCtl);
+}
+
 hipError_t res_alloc(Dims d, int nr, const ResPlan& pl, hipStream_t st, ResBuf& b) {
-  const size_t nk = (size_t)pl.nwg() * 2 * 2 * 4 * RES_NT;
-  const size_t nj = (size_t)pl.nwg() * (d.jp % 2 ? 2 : 1) * 2 * 2 * res_jn(pl.tk) * RES_NT;
-  const size_t ns = (size_t)2 * d.kp * nr;
+  const size_t nk = kwords(pl), nj = jwords(d, pl), ns = seam_floats(d, nr);
   hipError_t e = hipMalloc(&b.kslot, nk * sizeof(u64));
   if (e == hipSuccess) e = hipMalloc(&b.jslot, nj * sizeof(u64));
   if (e == hipSuccess) e = hipMalloc(&b.seam, ns * sizeof(float));

@@ -291,6 +291,13 @@ class LES:
         """SOR iteration form: tile_j = 0 two colour sweeps, else the fused launch's tile."""
         self._chk(lib().les_set_sor_tile(self.h, tile_j, tile_k), "set_sor_tile")
 
+    def solve_info(self):
+        """How the pressure solves run (les_get_solve_info); waits for the handle's stream."""
+        from ._lib import LesSolveInfo
+        s = LesSolveInfo()
+        self._chk(lib().les_get_solve_info(self.h, ctypes.byref(s)), "get_solve_info")
+        return {n: getattr(s, n) for n, _ in s._fields_}
+
     def time_kernel(self, which, reps=20):
         """Average milliseconds per launch of one kernel (HIP events on the handle's stream)."""
         out = ctypes.c_float()

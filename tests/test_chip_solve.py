@@ -32,6 +32,12 @@ def _same(a, b, names=FIELDS):
     assert np.abs(a.download("p")).max() > 0
 
 
+def _ran(h, solves, queued=0):
+    """The solves that were to run on the chip did, and in the form that was to be tested."""
+    i = h.solve_info()
+    assert (i["solves"], i["queued"], i["on_chip"], i["given_up"]) == (solves, queued, 1, 0), i
+
+
 # 1 workgroup; level blocks in one workgroup, the last partial; several along k; along j and k
 # with a partial top block; odd jp in one tile and in several; ip > 320; 9 levels a thread
 GRIDS = [(16, 12, 10), (31, 18, 17), (48, 48, 32), (150, 44, 61), (35, 27, 19), (20, 5, 7),
@@ -49,6 +55,8 @@ def test_chip_solve_equals_colour_sweeps(dims, dx):
     a.press_sor_solve()  # scatter, solve, gather
     b.press_sor_solve()
     _same(a, b, ("p",))
+    _ran(a, 5)
+    assert b.solve_info()["solves"] == 0 and not b.solve_info()["on_chip"]
     a.close()
     b.close()
 
@@ -62,10 +70,12 @@ def test_queue_form_equals_colour_sweeps(dims):
     a.run(1, 4)
     b.run(1, 4)
     _same(a, b)
+    _ran(a, 4, 4)
     assert lib().les_internal_sor_wait(a.h, ctypes.c_long(30000)) == 0
     a.run(5, 2)   # back to the resident form on the same buffers
     b.run(5, 2)
     _same(a, b)
+    _ran(a, 6, 4)
     a.close()
     b.close()
 
@@ -79,6 +89,7 @@ def test_two_handles_take_turns():
     hs[2].run(1, 8)
     for h in hs[:2]:
         _same(h, hs[2])
+        _ran(h, 8)
     for h in hs:
         h.close()
 
@@ -119,6 +130,7 @@ def test_early_exit_equals_colour_sweeps(dims, queue):
                 h.press_sor_solve()
             assert a.scalars() == b.scalars()
             _same(a, b, ("p",))
+        _ran(a, 7, 7 if queue else 0)
         a.close()
         b.close()
 
@@ -140,6 +152,7 @@ def test_queue_form_ends_with_the_exit():
         assert a.scalars() == b.scalars()
         assert n > 1 or a.scalars()["sor_iters"] == 3
         _same(a, b)
+    _ran(a, 8, 8)
     a.close()
     b.close()
 
@@ -232,3 +245,29 @@ def test_first_solves_while_another_thread_captures():
         _same(c, c0)
     for h in [a, b, c0] + cs:
         h.close()
+
+
+def test_handle_leaves_the_queue_form():
+    """16 solves in a row that find no room: the other forms from then on, the same values; one
+    resident solve in between starts the count anew."""
+    from les_halo_amd._lib import lib
+    dims = (48, 48, 32)
+    a, b = _handle(dims, 4, False), _handle(dims, 4, True)
+
+    def steps(first, last, wait):
+        assert lib().les_internal_sor_wait(a.h, ctypes.c_long(wait)) == 0
+        for n in range(first, last + 1):
+            a.run(n, 1)
+            a.sync()
+
+    steps(1, 10, -1)
+    steps(11, 11, 30000)
+    steps(12, 26, -1)
+    _ran(a, 26, 25)
+    steps(27, 32, -1)
+    i = a.solve_info()
+    assert (i["solves"], i["queued"], i["on_chip"], i["given_up"]) == (27, 26, 0, 1), i
+    b.run(1, 32)
+    _same(a, b)
+    a.close()
+    b.close()
