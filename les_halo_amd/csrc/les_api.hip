@@ -2078,8 +2078,8 @@ extern "C" int les_internal_sor_polls(les_handle* h, int polls) {
 }
 
 // Not part of the ABI: the number of tasks of the queue form.
-extern "C" int64_t les_internal_sor_tasks(int ip, int jp, int kp, int nmaxp) {
-  return (int64_t)res_queue_tasks(Dims{ip, jp, kp}, ((ip + 1) / 2 + 3) / 4 * 4, nmaxp);
+extern "C" int64_t les_internal_sor_tasks(int ip, int jp, int kp, int nwg, int nmaxp) {
+  return (int64_t)res_queue_tasks(Dims{ip, jp, kp}, ((ip + 1) / 2 + 3) / 4 * 4, nwg, nmaxp);
 }
 
 extern "C" int les_set_sor_tile(les_handle* h, int tile_j, int tile_k) {

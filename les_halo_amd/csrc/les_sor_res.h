@@ -18,14 +18,16 @@ struct ResPlan {
   __host__ __device__ int nwg() const { return njt * nkt; }
 };
 
-// The queue form: tasks of RES_NT groups per phase; the phases are the shifts, then one per sweep (odd
-// jp: two, the seam's copy first).  64 bits: any nmaxp is taken, and 500 000 iterations at
-// 300x300x90 pass 2^32 tasks.
-__host__ __device__ inline unsigned res_queue_blocks(const Dims& d, int nr) {
-  return ((unsigned)(nr / 4 * d.jp * d.kp) + RES_NT - 1) / RES_NT;
+// The queue form: at most one task a workgroup and phase, of RES_NT groups at least (the two fences of
+// a task cost more than its sweep does: with tasks of RES_NT groups 300x300x90 took 51 ms).
+// The phases are the shifts, then one per sweep (odd jp: two, the seam's copy first).  64 bits:
+// any nmaxp is taken.
+__host__ __device__ inline unsigned res_queue_blocks(const Dims& d, int nr, int nwg) {
+  const unsigned n = ((unsigned)(nr / 4 * d.jp * d.kp) + RES_NT - 1) / RES_NT;
+  return n < (unsigned)nwg ? n : (unsigned)nwg;
 }
-__host__ __device__ inline unsigned long long res_queue_tasks(const Dims& d, int nr, int nmaxp) {
-  return res_queue_blocks(d, nr) * (1ull + 2ull * nmaxp * (d.jp % 2 ? 2 : 1));
+__host__ __device__ inline unsigned long long res_queue_tasks(const Dims& d, int nr, int nwg, int nmaxp) {
+  return res_queue_blocks(d, nr, nwg) * (1ull + 2ull * nmaxp * (d.jp % 2 ? 2 : 1));
 }
 
 constexpr long RES_WAIT_TICKS = 30000;  // 0.3 ms of the 100 MHz clock

@@ -382,7 +382,7 @@ __device__ __forceinline__ void res_leave(const ResArgs& a, bool queued) {
 
 // The same solve through the task queue, on the split copy in device memory.  Phases in order:
 // the rhsav / pav shifts, then per sweep (odd jp: a copy of the two seam rows of the colour,
-// the values before the sweep, and) the sweep; nb tasks of RES_NT groups per phase.  A task of
+// the values before the sweep, and) the sweep; nb tasks per phase.  A task of
 // phase f starts when f * nb tasks have ended.  With the residual, the workgroup that adds the last
 // of an iteration's limbs decides before its task ends; after a stop the tasks left are void.
 template <bool RESID>
@@ -397,9 +397,10 @@ __device__ void res_queue(const ResArgs& a) {
   const int ng = sp.nr / 4, pl = sp.nr * sp.nj;
   const bool odd = d.jp & 1;
   const unsigned ngroups = (unsigned)(ng * d.jp * d.kp);
-  const unsigned nb = res_queue_blocks(d, sp.nr);
+  const unsigned nb = res_queue_blocks(d, sp.nr, a.pl.nwg());
+  const unsigned chunk = (ngroups + nb - 1) / nb;  // groups of a task
   const unsigned per = odd ? 2u : 1u;
-  const u64 ntask = res_queue_tasks(d, sp.nr, a.nmaxp);
+  const u64 ntask = res_queue_tasks(d, sp.nr, a.pl.nwg(), a.nmaxp);
   const float rsh = a.sub_rhsav ? a.sc->rhsav : 0.0f, psh = a.sub_pav ? a.sc->pav_carry : 0.0f;
   const float c2l = a.g.cn2l[0], c2s = a.g.cn2s[0], c3l = a.g.cn3l[0], c3s = a.g.cn3s[0];
   for (;;) {
@@ -427,8 +428,8 @@ __device__ void res_queue(const ResArgs& a) {
     const unsigned b = (unsigned)(n - ph * nb);
     ThreadAcc acc;
     acc.init();
-    const unsigned grp_id = b * RES_NT + threadIdx.x;
-    if (grp_id < ngroups) {
+    const unsigned end = min((b + 1u) * chunk, ngroups);
+    for (unsigned grp_id = b * chunk + threadIdx.x; grp_id < end; grp_id += RES_NT) {
       const int row = (int)(grp_id / (unsigned)ng), g4 = (int)(grp_id - (unsigned)(row * ng));
       const int kk = row / d.jp, j = 1 + row - kk * d.jp, k = 1 + kk;
       const int base = sp.nr * ((j - 1) + sp.nj * (k - 1)) + 4 * g4;
