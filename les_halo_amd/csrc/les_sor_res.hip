@@ -58,9 +58,10 @@ namespace les {
 
 constexpr int RES_WGMAX = 1024;  // (no device has that many CUs)
 struct ResCtl {
-  unsigned arrive, state, done, base;
-  unsigned failed;  // a wait was given up in this launch
-  unsigned queued, row;  // launches that took the queue form; of these the last in a row
+  unsigned arrive, state, done, queued;  // queued: launches that took the queue form
+  // low word: the launch's first tag; high: RES_FAILED, a wait was given up in this launch, and the
+  // number of launches in a row that took the queue form
+  unsigned long long base;
   ResHost* host;    // what the host is told
   unsigned long long ticket, tasks;  // the queue form's (phases x tasks can pass 32 bits)
   // the residual: workgroups that have added their exact sums, last iteration decided from them
@@ -81,6 +82,7 @@ constexpr int res_jn(int tk) { return (tk * 160 + RES_NT - 1) / RES_NT; }
 
 typedef unsigned long long u64;
 enum { RES_GO = 1, RES_QUEUE = 2 };
+constexpr u64 RES_FAILED = 1ull << 63;
 
 struct ResArgs {
   Dims d;
@@ -355,22 +357,21 @@ __device__ __forceinline__ void res_leave(const ResArgs& a, bool queued) {
   if (threadIdx.x != 0) return;
   const unsigned n = (unsigned)a.pl.nwg();
   if (atomicAdd(&a.ctl->done, 1u) != n - 1u) return;
-  const unsigned failed = agent_load(&a.ctl->failed), base = agent_load(&a.ctl->base);
-  const unsigned row = agent_load(&a.ctl->row);
-  if (queued || row) {  // (the host's memory is written only where something changes)
-    const unsigned total = agent_load(&a.ctl->queued) + (queued ? 1u : 0u), r = queued ? row + 1u : 0u;
-    agent_store(&a.ctl->queued, total);
-    agent_store(&a.ctl->row, r);
-    __hip_atomic_store(&a.ctl->host->queued, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(&a.ctl->host->row, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
-  if (failed) {
+  const u64 base = agent_load(&a.ctl->base);
+  unsigned row = (unsigned)(base >> 32) & 0x7fffffffu;
+  if (base & RES_FAILED) {
     for (int q = 0; a.slots && q < RED_SLOTS * NLIMB; ++q) agent_store(a.slots + q, (int64_t)0);
     agent_store(&a.sc->sor, __builtin_nanf(""));
     __hip_atomic_store(&a.ctl->host->failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    agent_store(&a.ctl->failed, 0u);
   }
-  agent_store(&a.ctl->base, base + 2u * (unsigned)a.nmaxp + 2u);
+  if (queued || row) {  // (the host's memory is written only where something changes)
+    const unsigned total = agent_load(&a.ctl->queued) + (queued ? 1u : 0u);
+    row = queued ? (row + 1u) & 0x7fffffffu : 0u;
+    agent_store(&a.ctl->queued, total);
+    __hip_atomic_store(&a.ctl->host->queued, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&a.ctl->host->row, row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  agent_store(&a.ctl->base, (u64)row << 32 | ((unsigned)base + 2u * (unsigned)a.nmaxp + 2u));
   agent_store(&a.ctl->arrive, 0u);
   agent_store(&a.ctl->ticket, (u64)0);
   agent_store(&a.ctl->tasks, (u64)0);
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
       }
     }
     sCtl[0] = st;
-    sCtl[1] = agent_load(&a.ctl->base);
+    sCtl[1] = (unsigned)agent_load(&a.ctl->base);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
@@ -906,7 +907,7 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
     }
   }
   if (budget <= 0) {
-    agent_store(&a.ctl->failed, 1u);
+    __hip_atomic_fetch_or(&a.ctl->base, RES_FAILED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __builtin_amdgcn_s_waitcnt(0);  // before this workgroup is counted as done
   }
   res_leave(a, false);
