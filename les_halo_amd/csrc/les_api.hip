@@ -1452,7 +1452,7 @@ int ensure_graph(les_handle* h) {
   if (h->graph) hipGraphDestroy(h->graph);
   h->gexec = nullptr;
   h->graph = nullptr;
-  (void)res_ready(h);  // no allocation inside the capture
+  (void)chip_solve(h, h->ph.pjuge > 0.0f);  // its buffers, if the step uses it: none are allocated in the capture
   h->graph_chip = false;
   int r;
   hipGraph_t gr = nullptr;

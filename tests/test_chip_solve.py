@@ -271,3 +271,24 @@ def test_handle_leaves_the_queue_form():
     _same(a, b)
     a.close()
     b.close()
+
+
+def test_no_memory_for_a_solve_that_is_not_used():
+    """A handle whose form was set by hand, or whose horizontal grid is not uniform, holds no face
+    slots, also after a captured step."""
+    from les_halo_amd import LES, inputs
+    dims = (48, 48, 32)
+    a = _handle(dims, 4, True)
+    b = LES(*dims, **common.REF_PHYS, omega=1.5, pjuge=0.0, nmaxp=4)
+    case = inputs.make_case(*dims, seed=5, hmax=20.0)
+    case["dx1"] = (case["dx1"] * np.linspace(1.0, 1.5, case["dx1"].size)).astype(np.float32)
+    d = case["dx1"]
+    case["dxs"] = (d[1:dims[0] + 2] / np.float32(2) + d[2:dims[0] + 3] / np.float32(2)).astype(np.float32)
+    b.load_case(case)
+    b.ifdata()
+    c = _handle(dims, 4, False)
+    for h, held in ((a, False), (b, False), (c, True)):
+        h.run(1, 4)
+        i = h.solve_info()
+        assert (i["face_bytes"] > 0, i["on_chip"] == 1, i["solves"] == 4) == (held,) * 3, i
+        h.close()
