@@ -415,8 +415,9 @@ typedef struct les_tuning {
   float stencil_ms[3];
 } les_tuning;
 int les_autotune(les_handle* h, int reps, les_tuning* out);
-/* Sets the SOR iteration form by hand (instead of the solve held on the chip): tile_j = 0 for two colour sweeps, else the fused launch
- * with tile_j (4, 8 or 16) rows of j and tile_k levels of k per workgroup. */
+/* Sets the SOR iteration form by hand (instead of the solve held on the chip, until les_autotune
+ * chooses again): tile_j = 0 for two colour sweeps, else the fused launch with tile_j (4, 8 or 16)
+ * rows of j and tile_k levels of k per workgroup. */
 int les_set_sor_tile(les_handle* h, int tile_j, int tile_k);
 /* How this handle's pressure solves run; waits for the handle's stream.  The solve held on the chip
  * needs all its workgroups resident together.  Where they are not within 0.3 ms (another program's

@@ -2186,6 +2186,13 @@ int tune_stencils(les_handle* h, int reps, les_tuning& best) {
 extern "C" int les_autotune(les_handle* h, int reps, les_tuning* out) {
   if (!h || reps < 1) return LES_E_INVALID;
   STAGE_BEGIN(h);
+  h->sor_form_set = false;  // the form is chosen here again
+  if (h->res_off) {         // (a row of solves in the queue form counts from here)
+    HIPCHK(h, hipStreamSynchronize(h->st));
+    if (h->rbuf.host) h->res_row0 = static_cast<volatile ResHost*>(h->rbuf.host)->row;
+    h->res_off = false;
+  }
+  h->graph_valid = false;
   sync_rhs(h);
   h->sp_p_current = false;  // the trials overwrite the split copy
   les_tuning best{};

@@ -292,3 +292,30 @@ def test_no_memory_for_a_solve_that_is_not_used():
         i = h.solve_info()
         assert (i["face_bytes"] > 0, i["on_chip"] == 1, i["solves"] == 4) == (held,) * 3, i
         h.close()
+
+
+def test_autotune_gives_the_form_back():
+    """After les_set_sor_tile, and after a row of solves in the queue form."""
+    from les_halo_amd._lib import lib
+    dims = (48, 48, 32)
+    a, b = _handle(dims, 4, False), _handle(dims, 4, True)
+    a.run(1, 2)
+    a.set_sor_tile(4, 5)
+    a.run(3, 2)
+    assert a.solve_info()["solves"] == 2 and not a.solve_info()["on_chip"]
+    a.autotune(2)
+    a.run(5, 2)
+    _ran(a, 4)
+    assert lib().les_internal_sor_wait(a.h, ctypes.c_long(-1)) == 0
+    a.run(7, 16)
+    assert a.solve_info()["given_up"]
+    a.autotune(2)
+    a.run(23, 3)
+    _ran(a, 23, 19)
+    assert lib().les_internal_sor_wait(a.h, ctypes.c_long(30000)) == 0
+    a.run(26, 2)
+    _ran(a, 25, 19)
+    b.run(1, 27)
+    _same(a, b)
+    a.close()
+    b.close()
