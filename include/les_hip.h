@@ -217,7 +217,9 @@ int les_step(les_handle* h, int n);
 int les_run(les_handle* h, int n0, int nsteps);
 /* Ensemble of independent members (handles of any sizes, each with its own state and
  * stream), advanced together: every step enqueues one graph launch of each member, step-major,
- * so the members' kernels run concurrently on the device.  No counterpart in the reference
+ * so the members' kernels run concurrently on the device (solves held on the chip share it: four
+ * at a time on a quarter of the CUs each, where a member's grid fits that; a grid that does not
+ * fit half the device runs its whole steps in turn).  No counterpart in the reference
  * (one domain per run); les_ensemble_run(e, n0, k) leaves every member as les_run(member, n0, k)
  * would.  Members keep their ownership (les_ensemble_destroy does not destroy them); mixed
  * precision members are not supported. */
@@ -420,7 +422,7 @@ int les_autotune(les_handle* h, int reps, les_tuning* out);
  * rows of j and tile_k levels of k per workgroup. */
 int les_set_sor_tile(les_handle* h, int tile_j, int tile_k);
 /* How this handle's pressure solves run; waits for the handle's stream.  The solve held on the chip
- * needs all its workgroups resident together.  Where they are not within 0.3 ms (another program's
+ * needs all its workgroups resident together.  Where they are not within 2 ms (another program's
  * kernels, masked CUs) a solve runs through a queue of tasks in device memory, several times
  * slower; after 16 of these in a row the handle takes the other forms (given_up). */
 typedef struct les_solve_info {
@@ -432,6 +434,7 @@ typedef struct les_solve_info {
   int given_up;     /* it fits but is no longer used: see above, or a solve failed (les_sync) */
   int64_t solves;   /* solves enqueued in that form */
   int64_t queued;   /* ... that ran through the queue */
+  int64_t shared;   /* ... that ran on part of the device, beside other handles' solves */
   int64_t face_bytes; /* device memory held for it */
 } les_solve_info;
 int les_get_solve_info(les_handle* h, les_solve_info* out);

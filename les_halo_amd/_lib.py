@@ -40,7 +40,7 @@ class LesTuning(ctypes.Structure):
 
 class LesSolveInfo(ctypes.Structure):
     _fields_ = [("on_chip", c_int), ("workgroups", c_int), ("rows", c_int), ("level_blocks", c_int),
-                ("levels", c_int), ("given_up", c_int), ("solves", c_int64), ("queued", c_int64),
+                ("levels", c_int), ("given_up", c_int), ("solves", c_int64), ("queued", c_int64), ("shared", c_int64),
                 ("face_bytes", c_int64)]
 
 

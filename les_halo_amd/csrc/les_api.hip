@@ -21,6 +21,9 @@
 
 using namespace les;
 
+// Cuts of the chip-resident solve: for the whole device, half of it and a quarter (ResTurn)
+constexpr int RES_CUTS = 3;
+
 struct les_handle {
   les_config cfg;
   Dims d;
@@ -76,8 +79,15 @@ struct les_handle {
                                 // sp_p_current and rhs_stale set)
   // The chip-resident solve (les_sor_res.hip): its cut of this grid (tk == 0: none) and its
   // device buffers, allocated by the first solve that uses them.
-  ResPlan rplan;
+  ResPlan rplan[RES_CUTS];  // on the whole device, on half and on a quarter of it
   ResBuf rbuf;
+  // the captured step in three: up to the solve, (the solve's arguments,) from it on
+  hipGraphExec_t gpre = nullptr, gpost = nullptr;
+  bool cap_split = false;  // ... is being captured
+  struct {
+    int sub_rhsav, sub_pav;
+    bool resid;
+  } cap{};
   bool sor_form_set = false;  // les_set_sor_tile chose the iteration's form
   bool capturing = false;     // the step is being captured into the handle's graph
   bool graph_chip = false;    // the captured step runs the chip-resident solve
@@ -85,12 +95,14 @@ struct les_handle {
   int res_polls = RES_POLLS;
   bool res_off = false;       // given up (RES_GIVE_UP, or a solve failed): the other forms are taken
   unsigned res_row0 = 0;      // ... of the row seen, what came before les_autotune
-  int64_t res_solves = 0;     // such solves enqueued
+  int64_t res_solves = 0;     // such solves enqueued, and those on part of the device
+  int64_t res_shared = 0;
   // for its turns with other handles (ResTurn, under its lock): the stream of the last launch with
   // such a solve, and an event recorded after that launch if res_rec
   hipStream_t res_st = nullptr;
   hipEvent_t res_ev = nullptr;
   bool res_rec = false;
+  unsigned res_clock = 0;     // ResTurn::clock then
   int ncu = 0;
   // workgroup shapes of the point-wise stencil kernels (les_autotune; 0 = 64 x 4)
   int shp_velnw = 0, shp_sm = 0, shp_visc = 0;
@@ -113,18 +125,24 @@ int fail(les_handle* h, int code, const std::string& msg) {
   } while (0)
 
 // The chip-resident solve wants all its workgroups on the device together, one per CU at most.
-// Handles whose solves could not be there at the same time take turns: while more than one of
-// them has used that solve and their workgroups together exceed the CUs, whoever launches next
-// makes its stream wait for the last launch of another one.  (Kernels of other programs are
-// not seen here; the solve itself falls back to its queue form when they keep it from fitting.)
+// Handles whose solves could not be there at the same time share it in four lanes of a quarter of the
+// CUs each.  While no other handle's solve is in flight a solve takes all four; else a cut of the
+// grid for two of them (with two handles) or one, where it fits, and waits for the last solve of
+// another handle on those lanes only.  A cut on a quarter takes 1.1 (48x48x32) to 2.1 times
+// (150x150x90) the time of the one on all CUs, and four of them run at once.  Grids that do not fit
+// half the device fill it with their other stages too: their whole step takes all lanes.
+// (Kernels of other programs are not seen here; the solve itself falls back to its queue form when
+// they keep it from fitting.)
 // A handle by itself records no events (4 us a step); when a second one comes, it records what the
 // first has launched so far, on the first one's stream: none of these streams is captured without
 // the lock, and a handle leaves the list before its streams are destroyed.
+constexpr int RES_LANES = 4;
 struct ResTurn {
   std::mutex m;
   std::vector<les_handle*> users;  // handles with chip-resident solves
   int wgs = 0;
-  les_handle* last = nullptr;
+  les_handle* lane[RES_LANES] = {};  // whose solve was last on it
+  unsigned used[RES_LANES] = {}, clock = 0;
 };
 constexpr int RES_DEVICES = 64;
 ResTurn g_turn[RES_DEVICES];
@@ -132,19 +150,19 @@ ResTurn g_turn[RES_DEVICES];
 // Allocates the chip-resident solve's buffers on first use; false: the grid does not fit or
 // there is no memory (the other forms of the solve serve it).
 bool res_ready(les_handle* h) {
-  if (h->rplan.tk == 0) return false;
+  if (h->rplan[0].tk == 0) return false;
   if (h->rbuf.ctl) return true;
   if (h->capturing) return false;
   ResTurn& T = g_turn[h->cfg.device];
   std::lock_guard<std::mutex> lock(T.m);
   if (!h->res_ev && hipEventCreateWithFlags(&h->res_ev, hipEventDisableTiming) != hipSuccess) h->res_ev = nullptr;
-  if (!h->res_ev || res_alloc(h->d, h->sp.nr, h->rplan, h->st, h->rbuf) != hipSuccess) {
+  if (!h->res_ev || res_alloc(h->d, h->sp.nr, h->rplan, RES_CUTS, h->st, h->rbuf) != hipSuccess) {
     (void)hipGetLastError();
-    h->rplan.tk = 0;
+    h->rplan[0].tk = 0;
     return false;
   }
   T.users.push_back(h);
-  T.wgs += h->rplan.nwg();
+  T.wgs += h->rplan[0].nwg();
   return true;
 }
 
@@ -153,8 +171,9 @@ void res_release(les_handle* h) {
     ResTurn& T = g_turn[h->cfg.device];
     std::lock_guard<std::mutex> lock(T.m);
     T.users.erase(std::find(T.users.begin(), T.users.end(), h));
-    T.wgs -= h->rplan.nwg();
-    if (T.last == h) T.last = nullptr;
+    T.wgs -= h->rplan[0].nwg();
+    for (auto& l : T.lane)
+      if (l == h) l = nullptr;
     res_free(h->rbuf);
   }
   if (h->res_ev) hipEventDestroy(h->res_ev);
@@ -184,31 +203,100 @@ void res_check(les_handle* h) {
   h->graph_valid = false;
 }
 
+// Under the lock: records what other handles launched while alone, and which of them are in flight.
+struct ResOthers {
+  bool share = false;  // their solves and this handle's exceed the device
+  std::vector<les_handle*> busy, unseen;  // unseen: on no lane so far
+  bool has(const les_handle* u) const { return std::find(busy.begin(), busy.end(), u) != busy.end(); }
+};
+hipError_t res_others(ResTurn& T, les_handle* h, ResOthers& o) {
+  o.share = T.users.size() > 1 && T.wgs > h->ncu;
+  if (!o.share) return hipSuccess;
+  for (les_handle* u : T.users) {
+    if (u == h || !u->res_st) continue;
+    const bool unseen = !u->res_rec;
+    if (unseen) {
+      const hipError_t e = hipEventRecord(u->res_ev, u->res_st);
+      if (e != hipSuccess) return e;
+      u->res_rec = true;
+    }
+    const hipError_t e = hipEventQuery(u->res_ev);
+    if (e == hipSuccess) continue;
+    (void)hipGetLastError();
+    if (e != hipErrorNotReady) return e;
+    o.busy.push_back(u);
+    if (unseen) o.unseen.push_back(u);
+  }
+  return hipSuccess;
+}
+// Two handles share only when they launch in alternation (or a few launches at a time): one that
+// starts behind a row of the other's solves, which have all lanes, runs after them in any case, and
+// alone.  With more there are others to run beside (a loop over eight handles of 48x48x32, each
+// enqueued 40 steps ahead: 0.83 ms a step of all, 1.8 each on all lanes).
+int res_cut(const ResTurn& T, const les_handle* h, const ResOthers& o) {
+  if (o.busy.empty()) return 0;
+  if (T.users.size() > 2) return h->rplan[2].tk > 0 ? 2 : h->rplan[1].tk > 0 ? 1 : 0;
+  const les_handle* u = o.busy[0];
+  const bool alternate = (int)(u->res_clock - h->res_clock) > 0 && T.clock - h->res_clock <= 4;
+  return alternate && h->rplan[1].tk > 0 ? 1 : 0;
+}
+// Under the lock: 'launch' enqueues work with a solve of h in that cut on stream st
+template <class Launch>
+hipError_t res_launch(ResTurn& T, les_handle* h, hipStream_t st, const ResOthers& o, int cut, Launch&& launch) {
+  int first = 0, n = RES_LANES >> cut;
+  if (o.share) {
+    // the lanes with the fewest solves in flight, of these the ones used longest ago
+    auto cost = [&](int l) { return T.lane[l] && T.lane[l] != h && o.has(T.lane[l]) ? 1 : 0; };
+    int best = RES_LANES + 1;
+    unsigned age = 0;
+    for (int l = 0; l < RES_LANES; l += n) {
+      int c = 0;
+      unsigned a = ~0u;
+      for (int q = l; q < l + n; ++q) {
+        c += cost(q);
+        a = std::min(a, T.lane[q] == h ? ~0u : T.clock - T.used[q]);
+      }
+      if (c < best || (c == best && a > age)) {
+        best = c;
+        age = a;
+        first = l;
+      }
+    }
+    // launches from before the lanes were used: all lanes come after this one, and it after them
+    if (!o.unseen.empty()) first = 0, n = RES_LANES;
+    hipError_t e = hipSuccess;
+    for (les_handle* u : o.busy) {
+      bool wait = std::find(o.unseen.begin(), o.unseen.end(), u) != o.unseen.end();
+      for (int l = first; l < first + n; ++l) wait = wait || T.lane[l] == u;
+      if (wait && (e = hipStreamWaitEvent(st, u->res_ev, 0)) != hipSuccess) return e;
+    }
+    h->res_clock = ++T.clock;
+  }
+  hipError_t e = launch(cut);
+  if (e == hipSuccess) {
+    ++h->res_solves;
+    h->res_shared += cut > 0;
+  }
+  h->res_st = st;
+  h->res_rec = false;
+  if (o.share) {
+    for (int l = first; l < first + n; ++l) {
+      T.lane[l] = h;
+      T.used[l] = T.clock;
+    }
+    if (e == hipSuccess) e = hipEventRecord(h->res_ev, st);
+    h->res_rec = e == hipSuccess;
+  }
+  return e;
+}
 // 'launch' enqueues work with a chip-resident solve of h on stream st, in its turn
 template <class Launch>
 hipError_t res_in_turn(les_handle* h, hipStream_t st, Launch&& launch) {
   ResTurn& T = g_turn[h->cfg.device];
   std::lock_guard<std::mutex> lock(T.m);
-  const bool share = T.users.size() > 1 && T.wgs > h->ncu;
-  if (share)
-    for (les_handle* u : T.users) {
-      if (u == h || !u->res_st) continue;
-      const bool unseen = !u->res_rec;
-      hipError_t e = unseen ? hipEventRecord(u->res_ev, u->res_st) : hipSuccess;
-      if (e == hipSuccess) u->res_rec = true;
-      if (e == hipSuccess && (unseen || u == T.last)) e = hipStreamWaitEvent(st, u->res_ev, 0);
-      if (e != hipSuccess) return e;
-    }
-  hipError_t e = launch();
-  T.last = h;
-  h->res_st = st;
-  h->res_rec = false;
-  if (e == hipSuccess) ++h->res_solves;
-  if (share && e == hipSuccess) {
-    e = hipEventRecord(h->res_ev, st);
-    h->res_rec = e == hipSuccess;
-  }
-  return e;
+  ResOthers o;
+  const hipError_t e = res_others(T, h, o);
+  return e != hipSuccess ? e : res_launch(T, h, st, o, res_cut(T, h, o), launch);
 }
 
 // Bounds table: lo/hi offsets relative to (0, ip, jp, kp) per dimension.
@@ -646,7 +734,8 @@ extern "C" int les_create(const les_config* cfg, les_handle** out) {
   }
   if (hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, cfg->device) != hipSuccess)
     return bail(LES_E_HIP);
-  if (cfg->device < RES_DEVICES) h->rplan = res_plan(h->d, h->sp.nr, h->ncu);
+  for (int q = 0; q < RES_CUTS && cfg->device < RES_DEVICES; ++q)
+    h->rplan[q] = res_plan(h->d, h->sp.nr, h->ncu >> q);
   h->resident_ok = cfg->precision == LES_PREC_FP32 && cfg->sum_order == LES_SUM_EXACT;
   if (cfg->sum_order == LES_SUM_REFERENCE) {
     const int nrt = (cfg->ip + 1) / 2;
@@ -661,7 +750,8 @@ extern "C" int les_create(const les_config* cfg, les_handle** out) {
 
 extern "C" int les_destroy(les_handle* h) {
   if (!h) return LES_OK;
-  if (h->gexec) hipGraphExecDestroy(h->gexec);
+  for (hipGraphExec_t x : {h->gexec, h->gpre, h->gpost})
+    if (x) hipGraphExecDestroy(x);
   if (h->graph) hipGraphDestroy(h->graph);
   if (h->st) hipStreamSynchronize(h->st);
   res_release(h);
@@ -1036,22 +1126,30 @@ bool use_split(const les_handle* h) {
 // choose it.
 bool chip_applies(const les_handle* h, bool resid) {
   return !(resid && seq_sums(h)) && h->sp.uniform && h->p_consistent && h->cn1_separable && h->split_ok &&
-         !h->sor_form_set && !h->res_off && h->cfg.nmaxp > 0 && h->rplan.tk > 0;
+         !h->sor_form_set && !h->res_off && h->cfg.nmaxp > 0 && h->rplan[0].tk > 0;
 }
 bool chip_solve(les_handle* h, bool resid) { return chip_applies(h, resid) && res_ready(h); }
 
+hipError_t enqueue_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_pav, bool resid, int cut) {
+  launch_sor_resident(h->st, h->d, grid_of(h), h->sp, ph, h->cfg.nmaxp, h->sc, sub_rhsav, sub_pav, h->ra[0],
+                      h->ra[1], resid ? h->rb.slots : nullptr, h->rplan[cut], h->rbuf, h->res_wait, h->res_polls);
+  return hipGetLastError();
+}
+
 int launch_chip_solve(les_handle* h, const Physics& ph, int sub_rhsav, int sub_pav, bool resid) {
-  auto go = [&]() {
-    launch_sor_resident(h->st, h->d, grid_of(h), h->sp, ph, h->cfg.nmaxp, h->sc, sub_rhsav, sub_pav,
-                        h->ra[0], h->ra[1], resid ? h->rb.slots : nullptr, h->rplan, h->rbuf, h->res_wait,
-                        h->res_polls);
-    return hipGetLastError();
-  };
-  if (h->capturing) {
+  if (h->cap_split) {  // (a captured step solves with the handle's own physics)
+    h->cap = {sub_rhsav, sub_pav, resid};
+    hipGraph_t gr = nullptr;
+    HIPCHK(h, hipStreamEndCapture(h->st, &gr));
+    const hipError_t e = hipGraphInstantiate(&h->gpre, gr, nullptr, nullptr, 0);
+    hipGraphDestroy(gr);
+    HIPCHK(h, e);
+    HIPCHK(h, hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal));
+  } else if (h->capturing) {
     h->graph_chip = true;
-    HIPCHK(h, go());
+    HIPCHK(h, enqueue_chip_solve(h, ph, sub_rhsav, sub_pav, resid, 0));
   } else {
-    HIPCHK(h, res_in_turn(h, h->st, go));
+    HIPCHK(h, res_in_turn(h, h->st, [&](int cut) { return enqueue_chip_solve(h, ph, sub_rhsav, sub_pav, resid, cut); }));
   }
   return LES_OK;
 }
@@ -1448,9 +1546,11 @@ int run_eager_prefix(les_handle* h, int n, int& nsteps, int& r) {
 // captures one step (n >= 2) of the handle into its graph, if not valid yet
 int ensure_graph(les_handle* h) {
   if (h->graph_valid) return LES_OK;
-  if (h->gexec) hipGraphExecDestroy(h->gexec);
+  for (hipGraphExec_t* x : {&h->gexec, &h->gpre, &h->gpost}) {
+    if (*x) hipGraphExecDestroy(*x);
+    *x = nullptr;
+  }
   if (h->graph) hipGraphDestroy(h->graph);
-  h->gexec = nullptr;
   h->graph = nullptr;
   (void)chip_solve(h, h->ph.pjuge > 0.0f);  // its buffers, if the step uses it: none are allocated in the capture
   h->graph_chip = false;
@@ -1479,10 +1579,44 @@ int ensure_graph(les_handle* h) {
   return LES_OK;
 }
 
-// one replay of the captured step (in its turn, when it runs the chip-resident solve)
+// the captured step again, in three
+hipError_t capture_split(les_handle* h) {
+  std::lock_guard<std::mutex> lock(g_turn[h->cfg.device].m);
+  hipError_t e = hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal);
+  if (e != hipSuccess) return e;
+  h->capturing = h->cap_split = true;
+  const int r = enqueue_step(h, 2);
+  h->capturing = h->cap_split = false;
+  hipGraph_t gr = nullptr;
+  e = hipStreamEndCapture(h->st, &gr);
+  if (e == hipSuccess && r) e = hipErrorStreamCaptureInvalidated;
+  if (e == hipSuccess) e = hipGraphInstantiate(&h->gpost, gr, nullptr, nullptr, 0);
+  if (gr) hipGraphDestroy(gr);
+  if (e == hipSuccess && !h->gpre) e = hipErrorStreamCaptureInvalidated;  // (the step has no such solve)
+  return e;
+}
+
+// One replay of the captured step.  With a chip-resident solve: in one, its solve on the whole
+// device, in its turn; or in three, its solve on the lanes it gets and the other stages beside
+// other handles' work.
 hipError_t replay_step(les_handle* h) {
   if (!h->graph_chip) return hipGraphLaunch(h->gexec, h->st);
-  return res_in_turn(h, h->st, [&]() { return hipGraphLaunch(h->gexec, h->st); });
+  ResTurn& T = g_turn[h->cfg.device];
+  {
+    std::lock_guard<std::mutex> lock(T.m);
+    ResOthers o;
+    hipError_t e = res_others(T, h, o);
+    if (e != hipSuccess) return e;
+    if (res_cut(T, h, o) == 0)
+      return res_launch(T, h, h->st, o, 0, [&](int) { return hipGraphLaunch(h->gexec, h->st); });
+  }
+  hipError_t e = h->gpost ? hipSuccess : capture_split(h);
+  if (e == hipSuccess) e = hipGraphLaunch(h->gpre, h->st);
+  if (e == hipSuccess)
+    e = res_in_turn(h, h->st, [&](int cut) {
+      return enqueue_chip_solve(h, h->ph, h->cap.sub_rhsav, h->cap.sub_pav, h->cap.resid, cut);
+    });
+  return e == hipSuccess ? hipGraphLaunch(h->gpost, h->st) : e;
 }
 
 // the host-side state a replay of the captured step leaves
@@ -1803,7 +1937,8 @@ extern "C" int les_ensemble_destroy(les_ensemble* e) {
 
 // Batched (when every member allows it): one launch per stage over all members.  Otherwise
 // every member's stream gets one graph launch per step, step-major, so the members' kernels
-// are in flight together and small members fill the device between the large ones.
+// are in flight together and small members fill the device between the large ones (replay_step:
+// with chip-resident solves, each on its lanes of the device).
 extern "C" int les_ensemble_run(les_ensemble* e, int n0, int nsteps) {
   if (!e || nsteps < 0) return LES_E_INVALID;
   if (batch_eligible(e)) {
@@ -2046,16 +2181,18 @@ extern "C" int les_get_solve_info(les_handle* h, les_solve_info* out) {
   const volatile ResHost* w = h->rbuf.host;
   res_check(h);
   out->on_chip = chip_applies(h, h->ph.pjuge > 0.0f) ? 1 : 0;
-  if (h->rplan.tk > 0) {
-    out->workgroups = h->rplan.nwg();
-    out->rows = h->rplan.rj;
-    out->level_blocks = h->rplan.ks;
-    out->levels = h->rplan.tk;
+  const ResPlan& pl = h->rplan[0];
+  if (pl.tk > 0) {
+    out->workgroups = pl.nwg();
+    out->rows = pl.rj;
+    out->level_blocks = pl.ks;
+    out->levels = pl.tk;
   }
   out->given_up = h->res_off ? 1 : 0;
   out->solves = h->res_solves;
   out->queued = w ? (int64_t)w->queued : 0;
-  out->face_bytes = h->rbuf.ctl ? (int64_t)res_bytes(h->d, h->sp.nr, h->rplan) : 0;
+  out->shared = h->res_shared;
+  out->face_bytes = h->rbuf.ctl ? (int64_t)res_bytes(h->d, h->sp.nr, h->rplan, RES_CUTS) : 0;
   return LES_OK;
 }
 

@@ -30,7 +30,9 @@ __host__ __device__ inline unsigned long long res_queue_tasks(const Dims& d, int
   return res_queue_blocks(d, nr, nwg) * (1ull + 2ull * nmaxp * (d.jp % 2 ? 2 : 1));
 }
 
-constexpr long RES_WAIT_TICKS = 30000;  // 0.3 ms of the 100 MHz clock
+// 2 ms of the 100 MHz clock: other handles' stencils hold CUs for some 0.1 ms at a time (with 0.3 ms a
+// few of 1000 solves of eight 150x150x90 handles took the queue form), and that form costs more.
+constexpr long RES_WAIT_TICKS = 200000;
 // So many solves in a row in the queue form, and the handle leaves this kernel: a few milliseconds
 // each at most, while one or two in a row are another kernel's that just ran.
 constexpr unsigned RES_GIVE_UP = 16;
@@ -55,9 +57,10 @@ struct ResBuf {
 };
 
 ResPlan res_plan(Dims d, int nr, int ncu);
-hipError_t res_alloc(Dims d, int nr, const ResPlan& pl, hipStream_t st, ResBuf& b);
+// buffers that serve every plan of pl[0..n) (one at a time: tags of launches only grow)
+hipError_t res_alloc(Dims d, int nr, const ResPlan* pl, int n, hipStream_t st, ResBuf& b);
 void res_free(ResBuf& b);
-size_t res_bytes(Dims d, int nr, const ResPlan& pl);  // device memory of res_alloc
+size_t res_bytes(Dims d, int nr, const ResPlan* pl, int n);  // device memory of res_alloc
 // nmaxp SOR iterations (press.f95:87-115) on the split copy sp.p / sp.r in place.  sub_rhsav: sp.r
 // holds the raw rhs; rhsav is taken off every value read and the result written to rout.
 // sub_pav: DevScalars::pav_carry is taken off every p value read.  resid_slots (RedBuf::slots, zero):

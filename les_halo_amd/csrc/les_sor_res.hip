@@ -955,19 +955,26 @@ ResPlan res_plan(Dims d, int nr, int ncu) {
 }
 
 namespace {
-size_t kwords(const ResPlan& pl) { return (size_t)pl.nwg() * 2 * 2 * 4 * RES_NT; }
-size_t jwords(Dims d, const ResPlan& pl) {
-  return (size_t)pl.nwg() * (d.jp % 2 ? 2 : 1) * 2 * 2 * res_jn(pl.tk) * RES_NT;
+size_t kwords(const ResPlan* pl, int n) {
+  size_t w = 0;
+  for (int q = 0; q < n; ++q) w = std::max(w, (size_t)pl[q].nwg() * 2 * 2 * 4 * RES_NT);
+  return w;
+}
+size_t jwords(Dims d, const ResPlan* pl, int n) {
+  size_t w = 0;
+  for (int q = 0; q < n; ++q)
+    w = std::max(w, (size_t)pl[q].nwg() * (d.jp % 2 ? 2 : 1) * 2 * 2 * res_jn(pl[q].tk) * RES_NT);
+  return w;
 }
 size_t seam_floats(Dims d, int nr) { return (size_t)2 * d.kp * nr; }
 }  // namespace
 
-size_t res_bytes(Dims d, int nr, const ResPlan& pl) {
-  return (kwords(pl) + jwords(d, pl)) * sizeof(u64) + seam_floats(d, nr) * sizeof(float) + sizeof(ResCtl);
+size_t res_bytes(Dims d, int nr, const ResPlan* pl, int n) {
+  return (kwords(pl, n) + jwords(d, pl, n)) * sizeof(u64) + seam_floats(d, nr) * sizeof(float) + sizeof(ResCtl);
 }
 
-hipError_t res_alloc(Dims d, int nr, const ResPlan& pl, hipStream_t st, ResBuf& b) {
-  const size_t nk = kwords(pl), nj = jwords(d, pl), ns = seam_floats(d, nr);
+hipError_t res_alloc(Dims d, int nr, const ResPlan* pl, int n, hipStream_t st, ResBuf& b) {
+  const size_t nk = kwords(pl, n), nj = jwords(d, pl, n), ns = seam_floats(d, nr);
   hipError_t e = hipMalloc(&b.kslot, nk * sizeof(u64));
   if (e == hipSuccess) e = hipMalloc(&b.jslot, nj * sizeof(u64));
   if (e == hipSuccess) e = hipMalloc(&b.seam, ns * sizeof(float));

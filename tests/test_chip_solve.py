@@ -319,3 +319,40 @@ def test_autotune_gives_the_form_back():
     _same(a, b)
     a.close()
     b.close()
+
+
+SHARED = [(96, 96, 20), (48, 48, 32), (147, 133, 61), (35, 27, 19), (150, 150, 90), (300, 300, 90)]
+
+
+@pytest.mark.parametrize("pjuge", [0.0, 1e-30])
+def test_handles_share_the_device(pjuge):
+    """Handles launched in alternation: solves on a half or a quarter of the CUs beside each other (the
+    grid of 8.1 M cells on all of them), the same values; then one of them alone again."""
+    from les_halo_amd import Ensemble
+    for dims in (SHARED[:2], SHARED):
+        print(dims, pjuge, flush=True)
+        hs = [_handle(d, 5, False, pjuge=pjuge) for d in dims]
+        refs = [_handle(d, 5, True, pjuge=pjuge) for d in dims]
+        E = Ensemble(hs, batched=False)
+        E.run(1, 2)
+        E.run(3, 12)
+        for h in hs:
+            h.press_sor_solve()
+        for h, r in zip(hs, refs):
+            r.run(1, 14)
+            r.press_sor_solve()
+            _same(h, r)
+            assert pjuge == 0.0 or h.scalars() == r.scalars()
+            i = h.solve_info()
+            assert i["solves"] == 15 and not i["given_up"], i
+        shared = [h.solve_info()["shared"] for h in hs]
+        assert all((n > 0) == (d != (300, 300, 90)) for d, n in zip(dims, shared)), shared
+        for h, r in ((hs[0], refs[0]), (hs[-1], refs[-1])):
+            h.run(15, 3)
+            h.sync()
+            r.run(15, 3)
+            _same(h, r)
+        assert [h.solve_info()["shared"] for h in hs] == shared
+        E.close()
+        for h in hs + refs:
+            h.close()
