@@ -2214,6 +2214,20 @@ extern "C" int les_internal_sor_polls(les_handle* h, int polls) {
   return LES_OK;
 }
 
+// Not part of the ABI: the cut of a grid for ncu CUs: levels per thread, level blocks, rows,
+// workgroups along j and k (levels 0: it does not fit).  A handle's own cut before its first solve.
+extern "C" int les_internal_sor_plan(int ip, int jp, int kp, int ncu, int out[5]) {
+  const ResPlan p = res_plan(Dims{ip, jp, kp}, ((ip + 1) / 2 + 3) / 4 * 4, ncu);
+  const int v[5] = {p.tk, p.ks, p.rj, p.njt, p.nkt};
+  std::copy(v, v + 5, out);
+  return LES_OK;
+}
+extern "C" int les_internal_sor_cut(les_handle* h, int ncu) {
+  if (!h || h->rbuf.ctl) return LES_E_STATE;
+  h->rplan[0] = res_plan(h->d, h->sp.nr, std::min(ncu, h->ncu));
+  return LES_OK;
+}
+
 // Not part of the ABI: the number of tasks of the queue form.
 extern "C" int64_t les_internal_sor_tasks(int ip, int jp, int kp, int nwg, int nmaxp) {
   return (int64_t)res_queue_tasks(Dims{ip, jp, kp}, ((ip + 1) / 2 + 3) / 4 * 4, nwg, nmaxp);

@@ -1,7 +1,7 @@
 """The SOR solve held on the chip (one launch, les_sor_res.hip) against the colour sweeps, bit for
 bit: cuts with one and several workgroups along j and k, partial top level blocks and last rows,
-colour rows with padding, odd jp (the periodic seam joins cells of one colour), the largest
-number of levels per thread; the queue form that serves it when its workgroups cannot all be
+colour rows with padding, odd jp (the periodic seam joins cells of one colour), every number of
+levels per thread with one and with several level blocks; the queue form that serves it when its workgroups cannot all be
 resident; two handles taking turns on one device; and the residual with the early exit."""
 import ctypes
 
@@ -356,3 +356,53 @@ def test_handles_share_the_device(pjuge):
         E.close()
         for h in hs + refs:
             h.close()
+
+
+# (levels per thread, several level blocks), grid, CUs to cut it for: every instance of the kernel, with
+# even and odd jp, several workgroups along j and k and a remainder along both
+CUTS = [((1, 0), (96, 20, 12), 96), ((1, 0), (61, 27, 12), 96), ((1, 1), (24, 44, 20), 48),
+        ((1, 1), (24, 27, 20), 24), ((2, 0), (391, 20, 33), 64), ((2, 0), (391, 27, 33), 96),
+        ((2, 1), (130, 20, 20), 12), ((2, 1), (35, 27, 33), 8), ((3, 0), (300, 44, 20), 64),
+        ((3, 0), (300, 61, 20), 64), ((3, 1), (48, 64, 33), 12), ((3, 1), (35, 27, 33), 4),
+        ((4, 0), (391, 20, 61), 48), ((4, 0), (391, 27, 33), 48), ((4, 1), (150, 44, 20), 12),
+        ((4, 1), (24, 27, 90), 4), ((5, 0), (391, 44, 33), 64), ((5, 0), (391, 61, 33), 96),
+        ((5, 1), (48, 64, 61), 12), ((5, 1), (61, 27, 33), 4), ((6, 0), (300, 64, 33), 32),
+        ((6, 0), (300, 61, 33), 32), ((6, 1), (96, 64, 33), 12), ((6, 1), (48, 27, 61), 4),
+        ((7, 0), (391, 44, 12), 12), ((7, 0), (391, 27, 12), 8), ((7, 1), (200, 44, 33), 16),
+        ((7, 1), (35, 27, 90), 4), ((8, 0), (200, 44, 61), 24), ((8, 0), (150, 61, 61), 24),
+        ((9, 0), (130, 64, 33), 12), ((9, 0), (150, 27, 33), 8), ((10, 0), (130, 64, 48), 16),
+        ((10, 0), (130, 61, 48), 16)]
+
+
+@pytest.mark.parametrize("kind, dims, ncu", CUTS)
+def test_every_cut_equals_colour_sweeps(kind, dims, ncu):
+    from les_halo_amd._lib import lib
+    for pjuge in (0.0, 1e-30):
+        print(kind, dims, ncu, pjuge, flush=True)
+        a, b = _handle(dims, 7, False, pjuge=pjuge), _handle(dims, 7, True, pjuge=pjuge)
+        assert lib().les_internal_sor_cut(a.h, ncu) == 0
+        a.run(1, 3)
+        b.run(1, 3)
+        _same(a, b)
+        assert pjuge == 0.0 or a.scalars() == b.scalars()
+        _ran(a, 3)
+        i = a.solve_info()
+        assert (i["levels"], int(i["level_blocks"] > 1)) == kind, i
+        a.close()
+        b.close()
+
+
+# grids near the largest that fit: 5 to 10 levels a thread on the whole device
+@pytest.mark.parametrize("dims, levels", [((166, 343, 68), 5), ((157, 525, 52), 6), ((194, 509, 66), 7),
+                                          ((283, 306, 78), 8), ((296, 328, 90), 10),
+                                          ((391, 224, 95), 10)])
+def test_large_grids_equal_colour_sweeps(dims, levels):
+    print(dims, flush=True)
+    a, b = _handle(dims, 3, False), _handle(dims, 3, True)
+    a.run(1, 2)
+    b.run(1, 2)
+    _same(a, b, ("p", "u", "rhs"))
+    _ran(a, 2)
+    assert a.solve_info()["levels"] == levels, a.solve_info()
+    a.close()
+    b.close()
