@@ -13,12 +13,12 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-7
 
 
-def _solve(dims, **kw):
+def _solve(dims, dx=4.0, dy=4.0, **kw):
     from les_halo_amd import LES, inputs
     from les_halo_amd.les import LES_PREC_MIXED
     L = LES(*dims, **common.REF_PHYS, omega=1.5, pjuge=0.0, nmaxp=50, precision=LES_PREC_MIXED,
             refine_tol=TOL, refine_max=40, refine_solver=1, **kw)
-    L.load_case(inputs.make_case(*dims, seed=9, hmax=20.0))
+    L.load_case(inputs.make_case(*dims, seed=9, hmax=20.0, dx=dx, dy=dy))
     L.ifdata()
     out = []
     for n in (1, 2, 3):
@@ -40,3 +40,12 @@ def test_multigrid_reaches_tolerance_in_few_iterations(dims):
 def test_another_relaxation_keeps_the_plain_pass():
     for s in _solve((40, 32, 20), refine_omega=1.5):
         assert s["resid_l2"] <= TOL, s
+
+
+@pytest.mark.parametrize("dx, dy", [(5.0, 3.0), (2.0, 10.0), (10.0, 2.0), (1.0, 20.0), (20.0, 1.0)])
+@pytest.mark.parametrize("dims", [(61, 34, 64), (24, 96, 20)])
+def test_multigrid_with_unequal_spacings(dims, dx, dy):
+    print(dims, dx, dy, flush=True)
+    for s in _solve(dims, dx, dy):
+        assert s["resid_l2"] <= TOL, s
+        assert s["cg_iters"] <= 40, s
