@@ -35,6 +35,9 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 # algorithmic FP32 bytes per interior cell-step: velnw 40 + velfg/feedbf/calc_sm 89 + visc/adam 88
 # + rhs 28 + 50 SOR iterations at 16 B (two 8 B colour sweeps) + pav/adj 12
 B_STEP = 1057
+# what the step moves with the solve held on the chip: p and rhs read and p written once per solve
+# instead of 16 B per iteration
+B_STEP_MOVED = 269
 VELFG_B_PER_CELL = 85          # velfg + feedbf (vel2 inlined)
 SOR_SWEEP_B_PER_CELL = 8       # one colour sweep: r p 4 + r rhs 2 + w p 2
 SOR_ITER_B_PER_CELL = 16       # one SOR iteration at press.f95's stage boundaries: two sweeps
@@ -398,10 +401,9 @@ def main():
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic_from_profiles(kname.replace(", false>", ">")), "kernel": kname,
-                "bytes_per_launch": bytes_launch, "avg_us": round(kern_ms * 1e3, 3),
-                "tile": [tuning["sor_tile_j"], tuning["sor_tile_k"]],
-                "tuned_iter_us": (round(tuning["sor_iter_ms"] * 1e3, 3)
-                                  if tuning["sor_iter_ms"] is not None else None)}
+                "bytes_per_launch": bytes_launch, "avg_us": round(kern_ms * 1e3, 3)}
+    if args.sor_tile:
+        roofline["tile"] = args.sor_tile
     if solve_us is not None:
         roofline["solve"] = {"kernel": "k_sor_resident", "us": round(solve_us, 1),
                              "bound": "exchange between CUs + instruction issue (on the chip)",
@@ -413,8 +415,9 @@ def main():
         roofline["compulsory_bytes_per_launch"] = compulsory
         roofline["compulsory_achieved"] = round(ach_c, 1)
         roofline["compulsory_frac"] = round(ach_c / HBM_PEAK_GBS, 4)
+    # (the bytes at the reference's stage boundaries, as the metric has them; the step's own below)
     step_hbm_frac = B_STEP * cells / (ms_per_step * 1e-3) / (HBM_PEAK_GBS * 1e9)
-    autotuned = {"sor_tile": [tuning["sor_tile_j"], tuning["sor_tile_k"]]}
+    autotuned = {"sor_tile": [tuning["sor_tile_j"], tuning["sor_tile_k"]]}  # (for solves not on the chip)
     if "stencil_shapes" in tuning:
         autotuned["stencil_shapes"] = tuning["stencil_shapes"]
 
@@ -428,6 +431,9 @@ def main():
                        "parallelism": "single domain, 1 GPU"},
             "step_hbm_frac": round(step_hbm_frac, 4), "step_bytes_per_cell": B_STEP,
             "autotuned": autotuned, "roofline": roofline}
+    if not args.sor_tile:
+        line["step_moved_bytes_per_cell"] = B_STEP_MOVED
+        line["step_moved_hbm_frac"] = round(step_hbm_frac * B_STEP_MOVED / B_STEP, 4)
     if args.tiled:
         line["tiled"] = tiled_bench(args.tiled, case)
     if args.adjoint:

@@ -402,7 +402,8 @@ int les_time_kernel(les_handle* h, int which, int reps, float* avg_ms);
  * workgroup tile (rows of j x levels of k), 'reps' iterations each, on this handle's grid, and
  * keeps the fastest (untuned handles use the two sweeps) for the solves that cannot be held on
  * the chip in one launch: where they can (uniform horizontal grid, mirror-image p halos, up to
- * about 9 million cells), that form is taken, tuned or not; then times the
+ * about 9 million cells with rows of up to 360, 4 million with rows of 440 to 512), that form is
+ * taken, tuned or not; then times the
  * velnw, calc_sm and viscous-term kernels with each of their workgroup shapes (64x4, 128x2,
  * 32x8, 256x1) and keeps the fastest of each.  Changes no simulation state (the arrays the
  * stencil trials update are saved and restored).  *out (may be NULL) receives the choice. */

@@ -1121,9 +1121,11 @@ bool use_split(const les_handle* h) {
 
 // The chip-resident solve (les_sor_res.hip) applies: a uniform horizontal grid that fits the
 // chip's LDS and registers, mirror-consistent p halos, cn1 of the separable form, no residual in
-// the reference's order of terms, and the form not set by hand.  Any parity of jp.  It is the
-// faster form wherever it fits (300x300x90: see the kernel's comment), so nothing is timed to
-// choose it.
+// the reference's order of terms, and the form not set by hand.  Any parity of jp.  A handle by
+// itself solves 2 to 3 times faster in it from 32x24x16 to the largest grids that fit (the kernel's
+// comment), several at once 1.2 to 1.5 times (ms a step of all, a loop over les_run, against the
+// fused iterations: 48x48x32 x 8 0.82 / 1.27, 96x96x60 x 16 2.18 / 3.36, 150x150x90 x 8 3.22 / 3.88),
+// so nothing is timed to choose it.
 bool chip_applies(const les_handle* h, bool resid) {
   return !(resid && seq_sums(h)) && h->sp.uniform && h->p_consistent && h->cn1_separable && h->split_ok &&
          !h->sor_form_set && !h->res_off && h->cfg.nmaxp > 0 && h->rplan[0].tk > 0;

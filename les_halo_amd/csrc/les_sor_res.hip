@@ -1,6 +1,8 @@
 // The whole red-black SOR solve of press.f95:87-115 in one launch, with p and rhs held on the
 // chip: 256 CUs have 160 KB of LDS and 512 KB of vector registers each, and 8 bytes a cell fit up
-// to about 9 million cells.
+// to about 9 million cells (rows of up to 360 cells; 8 million at 400).  Rows from 440 to 512 cells
+// fit up to about 4 million, longer ones not at all: a thread's words of a j face are fixed at rows
+// of 160 floats a level (res_jn), and a row has at most 64 groups.
 //
 // A thread owns a group of four consecutive entries of both colours' rows (j, k) over TK
 // consecutive levels (the colour-split layout of les_sor.hip): their p and rhs stay in its
@@ -39,15 +41,18 @@
 // goes to RES_QUEUE instead of RES_GO, once for all of them, and the same launch solves through
 // a task queue: tasks are taken in order from a counter, a task waits only for tasks before it,
 // and those are held by workgroups that are running, so it ends with any number of them
-// resident.  No input is overwritten before the decision.
+// resident.  No input is overwritten before the decision.  The queue form is slow (50 iterations at
+// 300x300x90 11.8 ms, 150x150x90 7.5, 32x24x16 1.4: two agent-scope fences a task and all workgroups
+// at two counters); the host is told how many solves took it and leaves this kernel after some.
 //
 // Bound: instruction issue and the exchange.  Per sweep at 300x300x90 (240 workgroups of 13 rows x
 // 9 levels): 2.0 us computing (77 vector instructions a group of four cells, two wavefronts per
 // SIMD), 0.9 us more with k faces only, 5.0 us with both; memory is read once and written once
 // per solve.  50 iterations, measured with the scatter and gather of p around them: 300x300x90
-// 592 us against 50 x 20.5 us for k_sor_iter; 150x150x90 282 against 50 x 11.7; 32x24x16 133
-// against 50 x 8.3; 147x133x61 (odd jp) about 250 against 100 x (9.2 + 4.9) + 50 x 4.6 in place.
-// With the residual (50 iterations): 1087, 694 and 299 us against 2109, 1471 and 1232 for the
+// 563 us against 50 x 20.5 us for k_sor_iter; 150x150x90 267 against 50 x 11.7; 32x24x16 (one
+// workgroup, no exchange: barriers and LDS latency) 133 against 50 x 8.3; the kernel alone at
+// 147x133x61 (odd jp) 227 against 100 x (9.2 + 4.9) + 50 x 4.6 in place.
+// With the residual (50 iterations): 1080, 700 and 300 us against 2140, 1440 and 1240 for the
 // residual-summing sweeps; what it adds is one all-workgroup hop an iteration (about 3 us, on the
 // smallest grid) and the sums' instructions.
 #include <algorithm>
@@ -918,8 +923,9 @@ __global__ __launch_bounds__(RES_NT) void k_sor_resident(ResArgs a) {
 // The cut with the least estimated time per sweep in us, fitted to the times of 40 cuts of
 // 150x150x90 and 96x96x60 and of smaller grids: per level 0.25 plus 0.045 for each wavefront of the
 // busiest SIMD; 0.9 for any faces, 0.28 per 1000 words of the k faces, 0.25 and 0.1 per 1000 words
-// for j faces, 0.15 where the XCDs' shares cut through a row of workgroups along k.  It prefers cuts about as high as they are long: 96x96x60 in 8 levels x 5 rows takes 1.7 us a sweep, in 1 x 32 2.3; 150x150x90
-// in 6 x 13 2.6, in 3 x 25 2.9.
+// for j faces, 0.15 where the XCDs' shares cut through a row of workgroups along k.  It prefers cuts
+// about as high as they are long: 96x96x60 in 8 levels x 5 rows takes 1.7 us a sweep, in 1 x 32 2.3;
+// 150x150x90 in 6 x 13 2.6, in 3 x 25 2.9.
 ResPlan res_plan(Dims d, int nr, int ncu) {
   ncu = std::min(ncu, RES_WGMAX);
   ResPlan best;
