@@ -1592,9 +1592,12 @@ hipError_t capture_split(les_handle* h) {
   hipGraph_t gr = nullptr;
   e = hipStreamEndCapture(h->st, &gr);
   if (e == hipSuccess && r) e = hipErrorStreamCaptureInvalidated;
+  if (e == hipSuccess && !h->gpre) e = hipErrorStreamCaptureInvalidated;  // (the step has no such solve)
   if (e == hipSuccess) e = hipGraphInstantiate(&h->gpost, gr, nullptr, nullptr, 0);
   if (gr) hipGraphDestroy(gr);
-  if (e == hipSuccess && !h->gpre) e = hipErrorStreamCaptureInvalidated;  // (the step has no such solve)
+  if (e == hipSuccess) return e;
+  if (h->gpre) hipGraphExecDestroy(h->gpre);
+  h->gpre = h->gpost = nullptr;
   return e;
 }
 
@@ -1604,16 +1607,19 @@ hipError_t capture_split(les_handle* h) {
 hipError_t replay_step(les_handle* h) {
   if (!h->graph_chip) return hipGraphLaunch(h->gexec, h->st);
   ResTurn& T = g_turn[h->cfg.device];
-  {
-    std::lock_guard<std::mutex> lock(T.m);
-    ResOthers o;
-    hipError_t e = res_others(T, h, o);
-    if (e != hipSuccess) return e;
-    if (res_cut(T, h, o) == 0)
-      return res_launch(T, h, h->st, o, 0, [&](int) { return hipGraphLaunch(h->gexec, h->st); });
+  for (bool split = true;; split = false) {  // (in one also if it cannot be captured in three)
+    {
+      std::lock_guard<std::mutex> lock(T.m);
+      ResOthers o;
+      const hipError_t e = res_others(T, h, o);
+      if (e != hipSuccess) return e;
+      if (!split || res_cut(T, h, o) == 0)
+        return res_launch(T, h, h->st, o, 0, [&](int) { return hipGraphLaunch(h->gexec, h->st); });
+    }
+    if (h->gpost || capture_split(h) == hipSuccess) break;
+    (void)hipGetLastError();
   }
-  hipError_t e = h->gpost ? hipSuccess : capture_split(h);
-  if (e == hipSuccess) e = hipGraphLaunch(h->gpre, h->st);
+  hipError_t e = hipGraphLaunch(h->gpre, h->st);
   if (e == hipSuccess)
     e = res_in_turn(h, h->st, [&](int cut) {
       return enqueue_chip_solve(h, h->ph, h->cap.sub_rhsav, h->cap.sub_pav, h->cap.resid, cut);

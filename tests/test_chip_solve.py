@@ -193,9 +193,9 @@ def test_polls_are_counted_per_sweep():
     together pass it many times over, ends like the sweeps' one."""
     from les_halo_amd._lib import lib
     dims = (48, 48, 32)
-    a, b = _handle(dims, 3000, False), _handle(dims, 3000, True)
-    # one sweep takes 2 us and a poll some tenths: a few thousand polls are far from any sweep's
-    assert lib().les_internal_sor_polls(a.h, 1 << 13) == 0
+    a, b = _handle(dims, 40000, False), _handle(dims, 40000, True)
+    # a sweep takes 2 us, a poll some tenths, and every sweep leaves some unanswered
+    assert lib().les_internal_sor_polls(a.h, 1 << 15) == 0
     for h in (a, b):
         h.step(1)
     a.sync()
