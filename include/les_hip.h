@@ -237,7 +237,8 @@ int les_ensemble_destroy(les_ensemble* e);
  * members; the fused SOR runs 4-row tiles with each member's tuned depth; calc_sm and visc use
  * the workgroup shape most members' autotuning chose), and the other stages are launched per
  * member inside the same graph.  Members must then outlive the ensemble.  Otherwise, and with
- * LES_ENSEMBLE_CONCURRENT, every member replays its own graph on its own stream.  The results
+ * LES_ENSEMBLE_CONCURRENT, every member replays its own graph on its own stream (the faster form
+ * where the members' solves are held on the chip; the batched one runs fused iterations).  The results
  * are the same bit for bit.  les_ensemble_batched returns 1 when the last run was batched. */
 enum { LES_ENSEMBLE_CONCURRENT = 0, LES_ENSEMBLE_BATCHED = 1 };
 int les_ensemble_set_mode(les_ensemble* e, int mode);
